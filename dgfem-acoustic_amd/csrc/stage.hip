@@ -623,6 +623,12 @@ __global__ __launch_bounds__((MfmaLaunch<T, D, P, SH>::KB), (MfmaLaunch<T, D, P,
     // than the caches hold passes before their next use: their loads and stores carry the
     // non-temporal hint, which leaves the caches to the neighbour traces and stage inputs (1-3% per
     // stage on the HBM-bound shapes)
+    // Without the compensated solution the accumulator of stages 0 and 1 is not stored: the stage
+    // inputs V1 = u + k1/2 and V2 = u + k2/2 already hold k1 and k2, so stage 2 (whose input is V2
+    // and whose output V3 replaces V1) forms A = u + ((V1 - u) + 2 (V2 - u) + k3) / 3 and stage 3
+    // adds k4/6. 13 state words per unknown and step are moved instead of 16, and u is rounded
+    // fewer times (A once instead of three times; V1 and V2 enter with weights 1/3 and 2/3).
+    // 2D order 2 FP64, 179,998 elements: 36.9 -> 35.4 us per stage; 3D order 3 FP64, 196,608: 131 -> 129.
     auto load_epi = [&]() {
     if (stage >= 1 && stage <= 3) {
 #pragma unroll
@@ -630,7 +636,9 @@ __global__ __launch_bounds__((MfmaLaunch<T, D, P, SH>::KB), (MfmaLaunch<T, D, P,
         if (tid + t * kBlock < nq * PV) {
           if (stage != 3 || CS) pu[t] = __builtin_nontemporal_load((const VT*)tile_at(U, e0, NP * ES, voff[t]));
           if (CS && stage == 3) plo[CS ? t : 0] = *(const uint2*)tile_at(Ulo, e0, NP * ES, voff[t]);
-          pa[t] = __builtin_nontemporal_load((const VT*)tile_at(Acc, e0, NP * ES, voff[t]));
+          if (CS || stage != 1)
+            pa[t] = __builtin_nontemporal_load(
+                (const VT*)tile_at(!CS && stage == 2 ? (const T*)Vout : (const T*)Acc, e0, NP * ES, voff[t]));
         }
     }
     };
@@ -818,11 +826,22 @@ __global__ __launch_bounds__((MfmaLaunch<T, D, P, SH>::KB), (MfmaLaunch<T, D, P,
       switch (stage) {
         case 0: {
           const VT u = *(const VT*)(sU + loff[t]);
-          __builtin_nontemporal_store(CS ? kq * s6 : u + kq * s6, pAcc);
+          if constexpr (CS) __builtin_nontemporal_store(kq * s6, pAcc);
           *pOut = u + kq * s2;
         } break;
-        case 1: __builtin_nontemporal_store(pa[t] + kq * s3, pAcc); *pOut = pu[t] + kq * s2; break;
-        case 2: __builtin_nontemporal_store(pa[t] + kq * s3, pAcc); *pOut = pu[t] + kq; break;
+        case 1:
+          if constexpr (CS) __builtin_nontemporal_store(pa[t] + kq * s3, pAcc);
+          *pOut = pu[t] + kq * s2;
+          break;
+        case 2:
+          if constexpr (CS) {
+            __builtin_nontemporal_store(pa[t] + kq * s3, pAcc);
+          } else {
+            const VT u = pu[t], v2 = *(const VT*)(sU + loff[t]);
+            __builtin_nontemporal_store(u + ((pa[t] - u) + (v2 - u) * (T)2 + kq) * s3, pAcc);
+          }
+          *pOut = pu[t] + kq;
+          break;
         case 3:
           if constexpr (CS) {
             const VT d = pa[t] + kq * s6;  // dt/6 (k1 + 2 k2 + 2 k3 + k4)
