@@ -416,7 +416,7 @@ struct MfmaCfg {
   static constexpr int RBP = rb_stride<T>(M::RB);
   static constexpr int NSB = 4 * TE * RBP > TE * LES ? 4 * TE * RBP : TE * LES;
   static constexpr size_t kLdsRest = sizeof(T) * (TE * LES + NSB + TE * NF * 4 + TE * 9) +
-                                     sizeof(int) * (NF * NPERM * NFP + NF * NFP) + (LO ? 16 * M::MB * M::NLO * 64 : 0);
+                                     sizeof(int) * NF * NPERM * NFP + (LO ? 16 * M::MB * M::NLO * 64 : 0);
   static constexpr size_t kLdsMax = 160 * 1024 - 512;
   // Operator fragments are staged in LDS whenever the whole workgroup footprint fits the 160 KiB
   // of a gfx950 CU (fewer resident workgroups, but no per-k-step global loads).
@@ -457,7 +457,16 @@ __global__ __launch_bounds__((MfmaLaunch<T, D, P, SH>::KB), (MfmaLaunch<T, D, P,
   // fields one LDS read; the LDS tiles use the same layout.
   static_assert(ES == D + 1 || ES == 4, "ES: the live field count");
   constexpr int NE = (4 * PV + kBlock - 1) / kBlock;        // state vectors per thread
-  constexpr int NI = (TE * NFF + kBlock - 1) / kBlock;      // face items per thread
+  // Face work: TPF threads share one element face, thread kk of them taking the face nodes kk,
+  // kk + TPF, ... (NI rounds), so that the face's connectivity, normal and flux coefficients are
+  // loaded and formed once per thread and tile, every LDS address is an invariant of the thread plus
+  // an immediate, and whole faces agree on being interior or boundary. The kernel is bound by vector
+  // instruction issue beside the MFMA chain (3D order 3: 425 per wave and tile, half of them here,
+  // when every face node looked up its own face); us per stage before -> after: 3D order 3, 196,608
+  // elements, FP32 85.1 -> 73.2, FP64 146 -> 124; 3D order 4, 115,000 elements, FP32 105 -> 94; 2D
+  // order 2 FP64, 179,998 elements, 38.2 -> 34.6 (event-timed launches).
+  constexpr int TPF = kBlock / (TE * NF);
+  constexpr int NI = (NFP + TPF - 1) / TPF;                 // face nodes per thread
   constexpr int NGEO = (TE * 9 + kBlock - 1) / kBlock;      // geometry values per thread
   constexpr int NFC = (TE * NF + kBlock - 1) / kBlock;      // element faces per thread
   typedef typename Mfma<T>::V V;
@@ -469,8 +478,7 @@ __global__ __launch_bounds__((MfmaLaunch<T, D, P, SH>::KB), (MfmaLaunch<T, D, P,
   __shared__ __attribute__((aligned(16))) T sB[NSB];
   __shared__ T sN[TE * NF][4];
   __shared__ T sG[TE][9];
-  __shared__ int sVmap[NF * NPERM * NFP];
-  __shared__ int sFmask[NF * NFP];
+  __shared__ uint32_t sVmap[NF * NPERM * NFP];  // byte offset of the neighbour's node in its element
   constexpr bool kALds = C::kALds;
   constexpr bool kCompact = C::kCompact;
   __shared__ T sA[kALds ? C::NAVS : 1];
@@ -495,8 +503,7 @@ __global__ __launch_bounds__((MfmaLaunch<T, D, P, SH>::KB), (MfmaLaunch<T, D, P,
   const T v0[3] = {(T)a.v0[0], (T)a.v0[1], (T)a.v0[2]};
   const int stage = a.stage;
   constexpr int nq = ES;  // the buffers hold exactly the live fields
-  for (int i = tid; i < NF * NPERM * NFP; i += kBlock) sVmap[i] = a.vmap[i];
-  for (int i = tid; i < NF * NFP; i += kBlock) sFmask[i] = a.fmask[i];
+  for (int i = tid; i < NF * NPERM * NFP; i += kBlock) sVmap[i] = (uint32_t)a.vmap[i] * (uint32_t)(ES * sizeof(T));
   if (kALds) {
     constexpr int NFULL = kCompact ? (MBF - 1) * KS * 64 : NAV;
     for (int i = tid; i < NFULL; i += kBlock) sA[i] = Af[i];
@@ -525,12 +532,26 @@ __global__ __launch_bounds__((MfmaLaunch<T, D, P, SH>::KB), (MfmaLaunch<T, D, P,
     loff[t] = v * VW + (v * VW / (NP * ES)) * C::PADV;
   }
 
+  // The thread's element face and its nodes' places in the LDS state tile. Threads beyond the last
+  // face (2D: 16 of 256) repeat it without storing.
+  static_assert(TPF >= 1, "every element face needs a thread");
+  const bool fact = TE * NF * TPF == kBlock || tid < TE * NF * TPF;
+  const int fp = fact ? tid / TPF : TE * NF - 1, kk = tid % TPF;
+  const int fj = fp % NF;
+  int fo[NI];
+#pragma unroll
+  for (int t = 0; t < NI; ++t) {
+    const int k = kk + t * TPF;
+    fo[t] = (fp / NF) * LES + a.fmask[fj * NFP + (k < NFP ? k : NFP - 1)] * ES;
+  }
+  auto has_node = [&](int t) { return fact && ((t + 1) * TPF <= NFP || kk + t * TPF < NFP); };
+
   // Software pipeline: while tile t is processed, tile t+1's state, geometry and face geometry,
-  // and the (neighbour, code) pairs of the thread's face items are in flight into registers; the
+  // and the (neighbour, code) pair of the thread's face are in flight into registers; the
   // neighbour traces of tile t+1 are gathered right after tile t's flux phase.
   VT pst[NE];
   T pgeo[NGEO], pfg[NFC][4];
-  int2 inc[NI], cnc[NI];
+  int2 inc, cnc;
   T iqp[NI][4];
   // value `rel` of an array of `per` values per element, at the tile starting at element e0 (32-bit
   // arithmetic unless BIG)
@@ -555,32 +576,17 @@ __global__ __launch_bounds__((MfmaLaunch<T, D, P, SH>::KB), (MfmaLaunch<T, D, P,
 #pragma unroll
         for (int c = 0; c < 4; ++c) pfg[t][c] = *tile_at(Fg, e0, NF * 4, (uint32_t)(idx * 4 + c));
     }
-#pragma unroll
-    for (int t = 0; t < NI; ++t) {
-      const int idx = tid + t * kBlock;
-      const int ej = (idx / NFF) * NF + (idx % NFF) / NFP;
-      inc[t] = idx < TE * NFF ? make_int2(*tile_at(a.nbr, e0, NF, (uint32_t)ej), *tile_at(a.code, e0, NF, (uint32_t)ej))
-                              : make_int2(-1, 0);
-    }
+    inc = make_int2(*tile_at(a.nbr, e0, NF, (uint32_t)fp), *tile_at(a.code, e0, NF, (uint32_t)fp));
   };
   auto gather = [&]() {
+    if (inc.x >= 0) {
+      const uint32_t* vm = sVmap + (inc.y & 0xffff) * NFP + kk;
+      // the neighbour element's base in 64 bits for BIG, else its 32-bit offset
+      const T* nb = BIG ? Vin + (uint64_t)(uint32_t)inc.x * (uint32_t)(NP * ES) : Vin;
+      const uint32_t nbo = BIG ? 0u : (uint32_t)inc.x * (uint32_t)(NP * ES * sizeof(T));
 #pragma unroll
-    for (int t = 0; t < NI; ++t) {
-      const int k = ((tid + t * kBlock) % NFF) % NFP;
-      if (inc[t].x >= 0) {
-        const uint32_t node = (uint32_t)sVmap[(inc[t].y & 0xffff) * NFP + k];
-        if constexpr (BIG) {
-          // the neighbour element's base in 64 bits, the node within it as a 32-bit offset
-          const T* nb = Vin + (uint64_t)(uint32_t)inc[t].x * (uint32_t)(NP * ES);
-          node_fields<ES>(byte_at(nb, node * (uint32_t)(ES * sizeof(T))), iqp[t]);
-        } else {
-          const uint32_t pi = (uint32_t)inc[t].x * (uint32_t)NP + node;
-          node_fields<ES>(byte_at(Vin, pi * (uint32_t)(ES * sizeof(T))), iqp[t]);
-        }
-      } else {
-#pragma unroll
-        for (int c = 0; c < 4; ++c) iqp[t][c] = (T)0;
-      }
+      for (int t = 0; t < NI; ++t)
+        if (has_node(t)) node_fields<ES>(byte_at(nb, nbo + vm[t * TPF]), iqp[t]);
     }
   };
 
@@ -646,57 +652,54 @@ __global__ __launch_bounds__((MfmaLaunch<T, D, P, SH>::KB), (MfmaLaunch<T, D, P,
     // chain: their epilogue operands are loaded later (below)
     constexpr bool kDefer = !kALds || MfmaLaunch<T, D, P, SH>::WAVES > 4 || MfmaLaunch<T, D, P, SH>::DEFER;
     if (!kDefer) load_epi();
-#pragma unroll
-    for (int t = 0; t < NI; ++t) cnc[t] = inc[t];
+    cnc = inc;
     const bool more = valid(it + bpx);
     if (more) prefetch((int64_t)(xcd * tpx + it + bpx) * TE);
     __syncthreads();
     // phase 2: nodal normal numerical fluxes scaled by sJ/|detJ| -> sB[(e*4 + q)*RB + jk]. All three face
-    // kinds share one branch-free form (no divergence between interior and boundary face nodes):
+    // kinds share one form:
     //   fl = A (F(qm) + F(qp)).n-with-speed-vne + H (qm - qp),   F(q).n = (vne p + rc2 v.n, vne v + p/rho n)
     // interior    qp = neighbour trace, A = 1/2, vne = v0.n, H = s c0/2      (Rusanov)
     // reflecting  qp = (p, v - 2 (v.n) n), A = 1/2, vne = v0.n, H = 0         (= n.F(p, v - (v.n) n))
     // absorbing   qp = (0, v - (v.n) n),   A = 1/4, vne = 0,    H = c0/4
     //             (= 1/4 [c0 p + rc2 v.n ; (p/rho + c0 v.n) n]; the qp part of F vanishes up to the
     //             rounding of v.n - (v.n)(n.n))
-    // the face nodes' LDS addresses are recomputed each tile (a few integer operations) rather than
-    // held across the tile loop: under register budgets of three or more waves per SIMD the
-    // compiler spilled them to scratch and reloaded them every tile, and in 1D/2D the registers
-    // saved raise the waves per SIMD (2D order 2 FP32: 5 -> 6, 10% faster); the 3D kernels without
-    // a budget keep them (the extra integer work slows the issue-bound order-5 kernel by 1%)
-    int ftid = tid;
-    if constexpr (MfmaLaunch<T, D, P, SH>::MINW >= 3 || D < 3) asm volatile("" : "+v"(ftid));
-#pragma unroll
-    for (int t = 0; t < NI; ++t) {
-      const int idx = ftid + t * kBlock;
-      if ((t + 1) * kBlock > TE * NFF && idx >= TE * NFF) continue;  // only the last round is partial
-      const int e = idx / NFF, jk = idx - e * NFF, j = jk / NFP;
-      const int ej = e * NF + j;
-      const int2 nc = cnc[t];
-      const T n[3] = {sN[ej][0], sN[ej][1], sN[ej][2]};
-      const T fs = sN[ej][3];
-      T qm[4];
-      node_fields<ES>(sU + e * LES + sFmask[jk] * ES, qm);
-      const T vn = v0[0] * n[0] + v0[1] * n[1] + v0[2] * n[2];
-      const T unm = qm[1] * n[0] + qm[2] * n[1] + qm[3] * n[2];
-      const bool inter = nc.x >= 0, refl = nc.x == -2;
-      const T gm = refl ? (T)2 : (T)1;
-      const T qp0 = inter ? iqp[t][0] : (refl ? qm[0] : (T)0);
-      T qpv[3];
-      for (int c = 0; c < 3; ++c) qpv[c] = inter ? iqp[t][1 + c] : qm[1 + c] - gm * unm * n[c];
-      const T unp = qpv[0] * n[0] + qpv[1] * n[1] + qpv[2] * n[2];
-      // the face scale fs is folded into A and H; sums before products:
-      //   fs fl_p = fs A (vne (pm + pp) + rc2 (un_m + un_p)) + fs H (pm - pp)
-      //   fs fl_v = fs A (vne (vm + vp) + (pm + pp)/rho n) + fs H (vm - vp)
+    // The face scale fs is folded into A and H, which belong to the face and are formed once per
+    // thread; sums before products:
+    //   fs fl_p = fs A (vne (pm + pp) + rc2 (vm + vp).n) + fs H (pm - pp)
+    //   fs fl_v = fs A (vne (vm + vp) + (pm + pp)/rho n) + fs H (vm - vp)
+    {
+      const T n[3] = {sN[fp][0], sN[fp][1], sN[fp][2]};
+      const T fs = sN[fp][3];
+      const bool inter = cnc.x >= 0, refl = cnc.x == -2;
       const T A = fs * ((inter || refl) ? (T)0.5 : (T)0.25);
-      const T H = fs * (inter ? (T)0.5 * ((nc.y >> 16) & 1 ? -c0 : c0) : (refl ? (T)0 : (T)0.25 * c0));
+      const T H = fs * (inter ? (T)0.5 * ((cnc.y >> 16) & 1 ? -c0 : c0) : (refl ? (T)0 : (T)0.25 * c0));
+      const T vn = v0[0] * n[0] + v0[1] * n[1] + v0[2] * n[2];
       const T Av = (inter || refl) ? A * vn : (T)0;
-      const T ps = qm[0] + qp0, pd = qm[0] - qp0;
-      const T Ap = A * irho * ps;
-      T fl[4];
-      fl[0] = Av * ps + (A * rc2) * (unm + unp) + H * pd;
-      for (int c = 0; c < 3; ++c) fl[1 + c] = Av * (qm[1 + c] + qpv[c]) + Ap * n[c] + H * (qm[1 + c] - qpv[c]);
-      for (int qq = 0; qq < 4; ++qq) sB[(e * 4 + qq) * RB + jk] = fl[qq];
+      const T Arc = A * rc2, Air = A * irho;
+      T* const fb = sB + (fp / NF) * 4 * RB + fj * NFP + kk;
+#pragma unroll
+      for (int t = 0; t < NI; ++t) {
+        T qm[4];
+        node_fields<ES>(sU + fo[t], qm);
+        if (!inter) {  // a boundary face: the ghost state takes the trace's place
+          const T un = (refl ? (T)2 : (T)1) * (qm[1] * n[0] + qm[2] * n[1] + qm[3] * n[2]);
+          iqp[t][0] = refl ? qm[0] : (T)0;
+          for (int c = 0; c < 3; ++c) iqp[t][1 + c] = qm[1 + c] - un * n[c];
+        }
+        const T ps = qm[0] + iqp[t][0], pd = qm[0] - iqp[t][0];
+        T vs[3], vd[3];
+        for (int c = 0; c < 3; ++c) {
+          vs[c] = qm[1 + c] + iqp[t][1 + c];
+          vd[c] = qm[1 + c] - iqp[t][1 + c];
+        }
+        const T Ap = Air * ps;
+        T fl[4];
+        fl[0] = Av * ps + Arc * (vs[0] * n[0] + vs[1] * n[1] + vs[2] * n[2]) + H * pd;
+        for (int c = 0; c < 3; ++c) fl[1 + c] = Av * vs[c] + Ap * n[c] + H * vd[c];
+        if (has_node(t))
+          for (int qq = 0; qq < 4; ++qq) fb[qq * RB + t * TPF] = fl[qq];
+      }
     }
     if (more) gather();  // next tile's neighbour traces, in flight during the MFMA phase
     __syncthreads();
