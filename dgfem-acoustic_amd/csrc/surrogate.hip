@@ -35,6 +35,8 @@ namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 struct Error : std::runtime_error {
   dgs_status st;
@@ -65,110 +67,246 @@ enum { EPI_STORE = 0, EPI_BIAS_ACT = 1, EPI_BIAS = 2, EPI_DACT = 3 };
 
 struct GemmArgs {
   int M, N, K;
-  const uint16_t* A;  // element (m, k) at A[m*sam + k*sak]
-  int64_t sam, sak;
-  const uint16_t* B;  // element (k, n) at B[n*sbn + k*sbk]
-  int64_t sbn, sbk;
+  int mrows;          // rows of the result that are stored (<= M)
+  const uint16_t* A;  // k-contiguous: element (m, k) at A[m*lda + k]; m-contiguous: A[k*lda + m]
+  int64_t lda;
+  const uint16_t* B;  // k-contiguous: element (k, n) at B[n*ldb + k]; n-contiguous: B[k*ldb + n]
+  int64_t ldb;
   const float* bias;  // [N]
-  float* pre;         // [M][ldc] pre-activation (written by BIAS_ACT, read by DACT)
+  float* pre;         // [M][ldc] pre-activation (written by BIAS_ACT when given, read by DACT)
   uint16_t* outb;     // [M][ldc] BF16 result
   float* outf;        // [M][ldc] FP32 result
   int ldc;
 };
 
-// C[M,N] = A[M,K] B[K,N] on v_mfma_f32_16x16x32_bf16. Workgroup: 4 waves, a 64x64 tile of C, each
-// wave a 32x32 quarter as 2x2 MFMA tiles; K advances 32 per step through LDS, where both operands
-// are stored k-contiguous ([row][k], rows padded to 40 values) so each lane's fragment is one
-// 16-byte read. Operand lane layout (probed on gfx950): A lane l holds A[l%16][8(l/16)+i],
-// B lane l holds B[8(l/16)+i][l%16]; accumulator register j of lane l is C[4(l/16)+j][l%16].
-// AT / BT: the operand is m- / n-contiguous in memory (else k-contiguous).
-// Shapes: M, N multiples of 64, K a multiple of 32 (checked on the host).
-template <bool AT, bool BT, int EPI>
-__global__ __launch_bounds__(256) void k_gemm(GemmArgs g) {
-  constexpr int LD = 40;
-  __shared__ __attribute__((aligned(16))) uint16_t sA[64 * LD];
-  __shared__ __attribute__((aligned(16))) uint16_t sB[64 * LD];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int m0 = blockIdx.y * 64, n0 = blockIdx.x * 64;
-  const int wr = (wave >> 1) * 32, wc = (wave & 1) * 32;
-  f32x4 acc[2][2];
-  for (int i = 0; i < 2; ++i)
-    for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0, 0, 0, 0};
-  for (int k0 = 0; k0 < g.K; k0 += 32) {
-    // stage the 64x32 operand tiles
-    if (!AT) {
-      const int r = tid >> 2, kq = (tid & 3) * 8;
-      *(uint4*)&sA[r * LD + kq] = *(const uint4*)&g.A[(int64_t)(m0 + r) * g.sam + (k0 + kq)];
-    } else {
-      const int r = tid & 63, kq = (tid >> 6) * 8;
-      for (int i = 0; i < 8; ++i) sA[r * LD + kq + i] = g.A[(int64_t)(m0 + r) * g.sam + (int64_t)(k0 + kq + i) * g.sak];
+// All products run on v_mfma_f32_16x16x32_bf16 with K ascending in steps of 32 from a zero
+// accumulator, so a result does not depend on the tile that computes it. Operand lane layout (probed
+// on gfx950): A lane l holds A[l%16][8(l/16)+i], B lane l holds B[8(l/16)+i][l%16]; accumulator
+// register j of lane l is C[4(l/16)+j][l%16]. Operands are staged in LDS k-contiguous ([row][k]), so
+// that each lane's fragment is one 16-byte read. Shapes: M, N, K multiples of 64 (checked on the
+// host), operands 16-byte aligned with lda and ldb multiples of 64.
+__device__ __forceinline__ f32x4 mma(const uint16_t* a, const uint16_t* b, f32x4 c) {
+  const bf16x8 va = __builtin_bit_cast(bf16x8, *(const u32x4*)a), vb = __builtin_bit_cast(bf16x8, *(const u32x4*)b);
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(va, vb, c, 0, 0, 0);
+}
+
+template <int EPI>
+__device__ __forceinline__ void gemm_store(const GemmArgs& g, int row, int col, float v) {
+  if (row >= g.mrows || col >= g.N) return;
+  const int64_t o = (int64_t)row * g.ldc + col;
+  if (EPI == EPI_STORE) {
+    g.outf[o] = v;
+  } else if (EPI == EPI_BIAS_ACT) {
+    const float p = v + g.bias[col];
+    if (g.pre) g.pre[o] = p;
+    g.outb[o] = f2bf(silu(p));
+  } else if (EPI == EPI_BIAS) {
+    g.outf[o] = v + g.bias[col];
+  } else {
+    g.outb[o] = f2bf(v * dsilu(g.pre[o]));
+  }
+}
+
+// Small tile: a 32x32 piece of C per workgroup, each of 4 waves a 16x16 quarter. A network layer of a
+// few hundred rows has only tens of 64x64 tiles for 256 CUs and is bound by memory latency, so the
+// tile is small and K goes through LDS in chunks of 256 (or its remainder, a multiple of 64), the next
+// two chunks' global loads in flight: one or two round trips cover a layer. 256 x 512 x 512: 10.1 ->
+// 4.6 us forward against 64x64 tiles loaded 32 k at a time without prefetch.
+// AT / BT: the operand is m- / n-contiguous in memory; a thread then loads 8 k-rows of 4 values and
+// transposes them in registers.
+constexpr int kSmall = 32, kChunk = 256, kSmallLd = kChunk + 8;
+struct Staged {
+  u32x4 v[4];
+};
+template <bool T>
+__device__ __forceinline__ void stage_load(const uint16_t* X, int64_t ld, int r0, int k0, int kc, Staged& s) {
+  const int tid = threadIdx.x;
+  if (!T) {
+    const uint16_t* p = X + (int64_t)(r0 + (tid >> 3)) * ld + k0 + (tid & 7) * 8;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (64 * i < kc) s.v[i] = *(const u32x4*)(p + 64 * i);
+  } else if ((tid >> 3) * 8 < kc) {
+    const uint16_t* p = X + (int64_t)(k0 + (tid >> 3) * 8) * ld + r0 + (tid & 7) * 4;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const u32x2 a = *(const u32x2*)(p + (2 * i) * ld), b = *(const u32x2*)(p + (2 * i + 1) * ld);
+      s.v[i] = u32x4{a.x, a.y, b.x, b.y};  // k-rows 2i and 2i+1, values 0..3 of each
     }
-    if (!BT) {
-      const int r = tid >> 2, kq = (tid & 3) * 8;
-      *(uint4*)&sB[r * LD + kq] = *(const uint4*)&g.B[(int64_t)(n0 + r) * g.sbn + (k0 + kq)];
+  }
+}
+template <bool T>
+__device__ __forceinline__ void stage_store(uint16_t* lds, int kc, const Staged& s) {
+  const int tid = threadIdx.x;
+  if (!T) {
+    uint16_t* p = lds + (tid >> 3) * kSmallLd + (tid & 7) * 8;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (64 * i < kc) *(u32x4*)(p + 64 * i) = s.v[i];
+  } else if ((tid >> 3) * 8 < kc) {
+    uint16_t* p = lds + (tid & 7) * 4 * kSmallLd + (tid >> 3) * 8;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {  // row j of the block: k-rows 0..7
+      uint32_t w[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const uint32_t lo = j < 2 ? s.v[i].x : s.v[i].y, hi = j < 2 ? s.v[i].z : s.v[i].w;
+        w[i] = j & 1 ? (lo >> 16) | (hi & 0xffff0000u) : (lo & 0xffffu) | (hi << 16);
+      }
+      *(u32x4*)(p + j * kSmallLd) = u32x4{w[0], w[1], w[2], w[3]};
+    }
+  }
+}
+
+template <bool AT, bool BT, int EPI>
+__device__ __forceinline__ void gemm_small(const GemmArgs& g, int bx, int by, uint16_t* sA, uint16_t* sB) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int m0 = by * kSmall, n0 = bx * kSmall;
+  const int wr = (wave >> 1) * 16, wc = (wave & 1) * 16;
+  const uint16_t* fa = sA + (wr + (lane & 15)) * kSmallLd + 8 * (lane >> 4);
+  const uint16_t* fb = sB + (wc + (lane & 15)) * kSmallLd + 8 * (lane >> 4);
+  f32x4 acc{0, 0, 0, 0};
+  Staged ra[2], rb[2];
+  auto load = [&](int k0, Staged& a, Staged& b) {
+    if (k0 >= g.K) return;
+    const int kc = min(kChunk, g.K - k0);
+    stage_load<AT>(g.A, g.lda, m0, k0, kc, a);
+    stage_load<BT>(g.B, g.ldb, n0, k0, kc, b);
+  };
+  auto chunk = [&](int k0, Staged& a, Staged& b) {
+    if (k0 >= g.K) return;
+    const int kc = min(kChunk, g.K - k0);
+    stage_store<AT>(sA, kc, a);
+    stage_store<BT>(sB, kc, b);
+    __syncthreads();
+    load(k0 + 2 * kChunk, a, b);
+    if (kc == kChunk) {
+#pragma unroll
+      for (int k = 0; k < kChunk; k += 32) acc = mma(fa + k, fb + k, acc);
     } else {
-      const int r = tid & 63, kq = (tid >> 6) * 8;
-      for (int i = 0; i < 8; ++i) sB[r * LD + kq + i] = g.B[(int64_t)(n0 + r) * g.sbn + (int64_t)(k0 + kq + i) * g.sbk];
+      for (int k = 0; k < kc; k += 32) acc = mma(fa + k, fb + k, acc);
     }
     __syncthreads();
-    bf16x8 a[2], b[2];
-    for (int i = 0; i < 2; ++i) {
-      const uint4 va = *(const uint4*)&sA[(wr + 16 * i + (lane & 15)) * LD + 8 * (lane >> 4)];
-      a[i] = __builtin_bit_cast(bf16x8, va);
-      const uint4 vb = *(const uint4*)&sB[(wc + 16 * i + (lane & 15)) * LD + 8 * (lane >> 4)];
-      b[i] = __builtin_bit_cast(bf16x8, vb);
+  };
+  load(0, ra[0], rb[0]);
+  load(kChunk, ra[1], rb[1]);
+  for (int k0 = 0; k0 < g.K; k0 += 2 * kChunk) {
+    chunk(k0, ra[0], rb[0]);
+    chunk(k0 + kChunk, ra[1], rb[1]);
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+    gemm_store<EPI>(g, m0 + wr + 4 * (lane >> 4) + r, n0 + wc + (lane & 15), acc[r]);
+}
+
+template <bool AT, bool BT, int EPI>
+__global__ __launch_bounds__(256) void k_gemm_small(GemmArgs g) {
+  __shared__ __attribute__((aligned(16))) uint16_t sA[kSmall * kSmallLd], sB[kSmall * kSmallLd];
+  gemm_small<AT, BT, EPI>(g, blockIdx.x, blockIdx.y, sA, sB);
+}
+
+// Large tile: BT x BT of C per workgroup (64 or 128), each of 4 waves a quarter, both operands
+// k-contiguous; K advances 64 per step through two LDS buffers with the next step's global loads in
+// registers. For layers with enough tiles to fill the chip, where the small tile would read every
+// operand value from L2 BT/32 times as often. Rows beyond M (N) repeat the last and are not stored.
+template <int BT, int EPI>
+__global__ __launch_bounds__(256) void k_gemm_large(GemmArgs g) {
+  constexpr int LD = 72, W = BT / 2, F = W / 16, NL = BT / 32;
+  __shared__ __attribute__((aligned(16))) uint16_t sA[2][BT * LD], sB[2][BT * LD];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int m0 = blockIdx.y * BT, n0 = blockIdx.x * BT;
+  const int wr = (wave >> 1) * W, wc = (wave & 1) * W;
+  f32x4 acc[F][F];
+#pragma unroll
+  for (int i = 0; i < F; ++i)
+#pragma unroll
+    for (int j = 0; j < F; ++j) acc[i][j] = f32x4{0, 0, 0, 0};
+  const int lr = tid >> 3, lk = (tid & 7) * 8;
+  const uint16_t *pa[NL], *pb[NL];
+#pragma unroll
+  for (int i = 0; i < NL; ++i) {
+    pa[i] = g.A + (int64_t)min(m0 + lr + 32 * i, g.M - 1) * g.lda + lk;
+    pb[i] = g.B + (int64_t)min(n0 + lr + 32 * i, g.N - 1) * g.ldb + lk;
+  }
+  u32x4 ra[NL], rb[NL];
+  auto load = [&](int k0) {
+#pragma unroll
+    for (int i = 0; i < NL; ++i) {
+      ra[i] = *(const u32x4*)(pa[i] + k0);
+      rb[i] = *(const u32x4*)(pb[i] + k0);
     }
-    for (int i = 0; i < 2; ++i)
-      for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
+  };
+  auto store = [&](int buf) {
+#pragma unroll
+    for (int i = 0; i < NL; ++i) {
+      *(u32x4*)&sA[buf][(lr + 32 * i) * LD + lk] = ra[i];
+      *(u32x4*)&sB[buf][(lr + 32 * i) * LD + lk] = rb[i];
+    }
+  };
+  load(0);
+  store(0);
+  __syncthreads();
+  for (int k0 = 0, buf = 0; k0 < g.K; k0 += 64, buf ^= 1) {
+    if (k0 + 64 < g.K) load(k0 + 64);
+#pragma unroll
+    for (int k = 0; k < 64; k += 32) {
+      bf16x8 a[F], b[F];
+#pragma unroll
+      for (int i = 0; i < F; ++i) {
+        const int o = (16 * i + (lane & 15)) * LD + k + 8 * (lane >> 4);
+        a[i] = __builtin_bit_cast(bf16x8, *(const u32x4*)&sA[buf][wr * LD + o]);
+        b[i] = __builtin_bit_cast(bf16x8, *(const u32x4*)&sB[buf][wc * LD + o]);
+      }
+#pragma unroll
+      for (int i = 0; i < F; ++i)
+#pragma unroll
+        for (int j = 0; j < F; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
+    }
+    if (k0 + 64 < g.K) store(buf ^ 1);
     __syncthreads();
   }
-  for (int i = 0; i < 2; ++i)
-    for (int j = 0; j < 2; ++j)
-      for (int r = 0; r < 4; ++r) {
-        const int row = m0 + wr + 16 * i + 4 * (lane >> 4) + r;
-        const int col = n0 + wc + 16 * j + (lane & 15);
-        const int64_t o = (int64_t)row * g.ldc + col;
-        const float v = acc[i][j][r];
-        if (EPI == EPI_STORE) {
-          g.outf[o] = v;
-        } else if (EPI == EPI_BIAS_ACT) {
-          const float p = v + g.bias[col];
-          g.pre[o] = p;
-          g.outb[o] = f2bf(silu(p));
-        } else if (EPI == EPI_BIAS) {
-          g.outf[o] = v + g.bias[col];
-        } else {
-          g.outb[o] = f2bf(v * dsilu(g.pre[o]));
-        }
-      }
+#pragma unroll
+  for (int i = 0; i < F; ++i)
+#pragma unroll
+    for (int j = 0; j < F; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        gemm_store<EPI>(g, m0 + wr + 16 * i + 4 * (lane >> 4) + r, n0 + wc + 16 * j + (lane & 15), acc[i][j][r]);
 }
 
 // z[r][f] = sin(2 pi B_f . x_r), z[r][F + f] = cos(2 pi B_f . x_r), rounded to BF16.
-__global__ void k_features(int n, int in, int F, const float* __restrict__ x, const float* __restrict__ Bm,
-                           uint16_t* __restrict__ z) {
+// Row r is taken from row idx[r] (when given) or min(r, m - 1) of x.
+__global__ void k_features(int n, int m, int in, int F, const int* __restrict__ idx, const float* __restrict__ x,
+                           const float* __restrict__ Bm, uint16_t* __restrict__ z) {
   const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (i >= (int64_t)n * F) return;
   const int r = (int)(i / F), f = (int)(i % F);
+  const int64_t xr = idx ? idx[r] : min(r, m - 1);
   float a = 0;
-  for (int d = 0; d < in; ++d) a += Bm[f * in + d] * x[r * in + d];
+  for (int d = 0; d < in; ++d) a += Bm[f * in + d] * x[xr * in + d];
   a *= 6.283185307179586f;
   z[(int64_t)r * 2 * F + f] = f2bf(sinf(a));
   z[(int64_t)r * 2 * F + F + f] = f2bf(cosf(a));
 }
 
 // Relative squared error per sample: loss_r = w_r sum_j (y - t)^2, w_r = 1 / (n |t_r|^2);
-// dY = 2 w_r (y - t) rounded to BF16. One workgroup per sample row.
+// dY = 2 w_r (y - t) rounded to BF16. One workgroup per sample row. With idx, row r's target and
+// weight are row idx[r] of the resident set, the weight divided by the batch size so that the
+// minibatch loss is the mean of W_r |y_r - t_r|^2.
 __global__ __launch_bounds__(256) void k_loss(int N, const float* __restrict__ y, const float* __restrict__ t,
-                                              const float* __restrict__ w, uint16_t* __restrict__ dy,
-                                              float* __restrict__ loss_row) {
+                                              const float* __restrict__ w, const int* __restrict__ idx,
+                                              uint16_t* __restrict__ dy, float* __restrict__ loss_row) {
   __shared__ float red[256];
   const int r = blockIdx.x;
+  const int64_t tr = idx ? idx[r] : r;
+  const float wr = idx ? w[tr] / (float)(int)gridDim.x : w[tr];
   float s = 0;
   for (int j = threadIdx.x; j < N; j += 256) {
     const int64_t o = (int64_t)r * N + j;
-    const float d = y[o] - t[o];
+    const float d = y[o] - t[tr * N + j];
     s += d * d;
-    dy[o] = f2bf(2.0f * w[r] * d);
+    dy[o] = f2bf(2.0f * wr * d);
   }
   red[threadIdx.x] = s;
   __syncthreads();
@@ -176,16 +314,53 @@ __global__ __launch_bounds__(256) void k_loss(int N, const float* __restrict__ y
     if (threadIdx.x < k) red[threadIdx.x] += red[threadIdx.x + k];
     __syncthreads();
   }
-  if (threadIdx.x == 0) loss_row[r] = w[r] * red[0];
+  if (threadIdx.x == 0) loss_row[r] = wr * red[0];
 }
 
-// db[n] = sum_m d[m][n] over BF16 rows.
-__global__ void k_colsum(int M, int N, const uint16_t* __restrict__ d, float* __restrict__ db) {
-  const int n = blockIdx.x * blockDim.x + threadIdx.x;
-  if (n >= N) return;
-  float s = 0;
-  for (int m = 0; m < M; ++m) s += bf2f(d[(int64_t)m * N + n]);
-  db[n] = s;
+// db[n] = sum_m d[m][n] over BF16 rows, 64 columns per workgroup, m ascending. The sum is one serial
+// chain per column; what it waited for was a dependent memory round trip every few rows (31 us at 256
+// x 512), so 256 rows at a time come in coalesced 16-byte loads through LDS (s: 256 * 64 values).
+constexpr int kSumCols = 64, kSumRows = 256;
+__device__ __forceinline__ void colsum(int M, int N, const uint16_t* __restrict__ d, float* __restrict__ db, int n0,
+                                       uint16_t* s) {
+  const int tid = threadIdx.x;
+  float sum = 0;
+  for (int m0 = 0; m0 < M; m0 += kSumRows) {
+    u32x4 v[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int m = m0 + 32 * i + (tid >> 3);
+      if (m < M) v[i] = *(const u32x4*)(d + (int64_t)m * N + n0 + (tid & 7) * 8);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (m0 + 32 * i + (tid >> 3) < M) *(u32x4*)(s + (32 * i + (tid >> 3)) * kSumCols + (tid & 7) * 8) = v[i];
+    __syncthreads();
+    if (tid < kSumCols) {
+      const int rows = min(kSumRows, M - m0);
+#pragma unroll 16
+      for (int m = 0; m < rows; ++m) sum += bf2f(s[m * kSumCols + tid]);
+    }
+  }
+  if (tid < kSumCols) db[n0 + tid] = sum;
+}
+
+// Backward pass of one layer in one launch: the workgroups take the tiles of dX = (d W) silu'(pre)
+// (nx of them, none for the first layer), of dW = d^T x, and the bias gradient's column groups.
+__global__ __launch_bounds__(256) void k_backward(GemmArgs dx, int nx, GemmArgs dw, int nw, int rows, float* db) {
+  __shared__ __attribute__((aligned(16))) uint16_t sh[2 * kSmall * kSmallLd];
+  static_assert(2 * kSmall * kSmallLd >= kSumRows * kSumCols, "the column sums share the tiles' LDS");
+  const int b = blockIdx.x;
+  if (b < nx) {
+    const int cols = dx.N / kSmall;
+    gemm_small<false, true, EPI_DACT>(dx, b % cols, b / cols, sh, sh + kSmall * kSmallLd);
+  } else if (b < nx + nw) {
+    const int t = b - nx, cols = dw.N / kSmall;
+    gemm_small<true, true, EPI_STORE>(dw, t % cols, t / cols, sh, sh + kSmall * kSmallLd);
+  } else {
+    colsum(rows, dw.M, dw.A, db, (b - nx - nw) * kSumCols, sh);
+  }
 }
 
 // sum of n values into out[0] (one workgroup)
@@ -221,18 +396,6 @@ __global__ void k_adam(int64_t n, float* __restrict__ p, uint16_t* __restrict__ 
 __global__ void k_tobf(int64_t n, const float* __restrict__ p, uint16_t* __restrict__ pb) {
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
     pb[i] = f2bf(p[i]);
-}
-
-// rows idx[r] of (x, t, w) -> batch buffers; the weight is divided by the batch size so that the
-// minibatch loss is the mean of W_r |y_r - t_r|^2
-__global__ void k_gather(int n, int in, int N, const int* __restrict__ idx, const float* __restrict__ X,
-                         const float* __restrict__ T, const float* __restrict__ W, float* __restrict__ x,
-                         float* __restrict__ t, float* __restrict__ w) {
-  const int r = blockIdx.x;
-  const int64_t s = idx[r];
-  for (int j = threadIdx.x; j < N; j += blockDim.x) t[(int64_t)r * N + j] = T[s * N + j];
-  if (threadIdx.x < in) x[r * in + threadIdx.x] = X[s * in + threadIdx.x];
-  if (threadIdx.x == 0) w[r] = W[s] / (float)n;
 }
 
 }  // namespace
@@ -298,33 +461,37 @@ dgs_status guarded(Net* n, F&& f) {
   }
 }
 
-template <bool AT, bool BT, int EPI>
+void check_gemm(const GemmArgs& g) {
+  if (g.M % 64 || g.N % 64 || g.K % 64 || g.M <= 0 || g.N <= 0 || g.K <= 0)
+    throw Error(DGS_ERR_INVALID, "GEMM shape must be multiples of 64");
+}
+
+// C = A B with both operands k-contiguous (the forward pass): the largest tile whose grid still
+// fills the chip.
+template <int EPI>
 void gemm(Net& n, GemmArgs g) {
-  if (g.M % 64 || g.N % 64 || g.K % 32 || g.M <= 0 || g.N <= 0 || g.K <= 0)
-    throw Error(DGS_ERR_INVALID, "GEMM shape must be M, N multiples of 64 and K a multiple of 32");
-  hipLaunchKernelGGL((k_gemm<AT, BT, EPI>), dim3(g.N / 64, g.M / 64), dim3(256), 0, n.s, g);
+  check_gemm(g);
+  auto grid = [&](int t) { return dim3((g.N + t - 1) / t, (g.M + t - 1) / t); };
+  auto tiles = [&](int t) { return (int64_t)grid(t).x * grid(t).y; };
+  if (tiles(128) >= 192) hipLaunchKernelGGL((k_gemm_large<128, EPI>), grid(128), dim3(256), 0, n.s, g);
+  else if (tiles(64) >= 384) hipLaunchKernelGGL((k_gemm_large<64, EPI>), grid(64), dim3(256), 0, n.s, g);
+  else hipLaunchKernelGGL((k_gemm_small<false, false, EPI>), grid(kSmall), dim3(256), 0, n.s, g);
   DGS_HIP(hipGetLastError());
 }
 
-// Device buffers of one forward pass: inputs x [rows][in], features z, per hidden layer l the BF16
-// activations h(l) and FP32 pre-activations pre(l), output y [rows][out].
+// Device buffers of one forward pass: inputs x [m][in] (padded to whole tiles with copies of the
+// last row, or rows idx[r] of x), features z, per hidden layer l the BF16 activations h(l) and (for
+// a backward pass) FP32 pre-activations pre(l), output y [m][out].
 struct Pass {
   const float* x;
+  int m;                       // rows of x and y
+  const int* idx = nullptr;
   uint16_t* z;
   uint16_t* h[2];  // hidden layer l writes h[l % 2] (when not per layer)
-  float* pre;      // one buffer for every hidden layer (when not per layer)
   const std::vector<uint16_t*>* hl = nullptr;  // per-layer buffers (training keeps them for backward)
   const std::vector<float*>* prel = nullptr;
   float* y;
 };
-
-// rows [0, mp) of dst take source rows min(r, m - 1) of x (padding with copies of the last row)
-__global__ void k_pad_rows(const float* __restrict__ x, int m, int mp, int in, float* __restrict__ dst) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= mp * in) return;
-  const int r = i / in, c = i - r * in;
-  dst[i] = x[(int64_t)min(r, m - 1) * in + c];
-}
 
 // Device address of `scratch` on device dev, looked up once per device with that device current.
 std::mutex g_scratch_mu;
@@ -345,24 +512,30 @@ unsigned char* scratch_base(int dev) {
   return g_scratch[dev];
 }
 
-// Layout of one forward pass of mp rows in the scratch array (256-byte aligned pieces); returns the
-// bytes needed.
+size_t aligned256(size_t bytes) { return (bytes + 255) / 256 * 256; }
+
+// Layout of one forward pass of mp rows in the scratch array (256-byte aligned pieces: features and
+// two layers' activations; inputs and outputs stay in the caller's memory); returns the bytes needed.
 size_t scratch_layout(const Net& n, int mp, unsigned char* base, Pass* b) {
   const dgs_config& k = n.cfg;
-  size_t off = 0;
-  auto take = [&](size_t bytes) {
-    unsigned char* p = base ? base + off : nullptr;
-    off += (bytes + 255) / 256 * 256;
-    return p;
-  };
-  float* x = (float*)take((size_t)mp * k.in_dim * sizeof(float));
-  b->x = x;
-  b->z = (uint16_t*)take((size_t)mp * 2 * k.n_freq * sizeof(uint16_t));
-  b->h[0] = (uint16_t*)take((size_t)mp * k.width * sizeof(uint16_t));
-  b->h[1] = (uint16_t*)take((size_t)mp * k.width * sizeof(uint16_t));
-  b->pre = (float*)take((size_t)mp * k.width * sizeof(float));
-  b->y = (float*)take((size_t)mp * k.out_dim * sizeof(float));
-  return off;
+  const size_t z = aligned256((size_t)mp * 2 * k.n_freq * sizeof(uint16_t));
+  const size_t h = aligned256((size_t)mp * k.width * sizeof(uint16_t));
+  if (base) {
+    b->z = (uint16_t*)base;
+    b->h[0] = (uint16_t*)(base + z);
+    b->h[1] = (uint16_t*)(base + z + h);
+  }
+  return z + 2 * h;
+}
+
+// The networks the allocation-free pass takes: those whose 64 rows of inputs, features, activations,
+// FP32 pre-activations and outputs fit the scratch array.
+bool scratch_takes(const Net& n) {
+  const dgs_config& k = n.cfg;
+  const size_t f = sizeof(float);
+  return aligned256(64 * (size_t)k.in_dim * f) + scratch_layout(n, 64, nullptr, nullptr) +
+             aligned256(64 * (size_t)k.width * f) + aligned256(64 * (size_t)k.out_dim * f) <=
+         kScratchBytes;
 }
 
 void check_batch(const Net& n, int rows) {
@@ -370,42 +543,44 @@ void check_batch(const Net& n, int rows) {
     throw Error(DGS_ERR_INVALID, "batch rows must be a positive multiple of 64 up to max_batch");
 }
 
-// forward pass of `rows` rows already in n.x; output in n.y
-void forward(Net& n, int rows);
+// forward pass of `rows` rows (a multiple of 64)
 void forward(Net& n, int rows, const Pass& b) {
   const int F = n.cfg.n_freq, in = n.cfg.in_dim;
   const int64_t tot = (int64_t)rows * F;
-  hipLaunchKernelGGL(k_features, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, n.s, rows, in, F, b.x, n.Bm, b.z);
+  hipLaunchKernelGGL(k_features, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, n.s, rows, b.m, in, F, b.idx, b.x,
+                     n.Bm, b.z);
   DGS_HIP(hipGetLastError());
   const uint16_t* a = b.z;
   for (int l = 0; l < n.L; ++l) {
     GemmArgs g{};
-    g.M = rows;
+    g.M = g.mrows = rows;
     g.N = n.dout[l];
     g.K = n.din[l];
     g.A = a;
-    g.sam = n.din[l];
-    g.sak = 1;
+    g.lda = n.din[l];
     g.B = n.Pb + n.woff[l];
-    g.sbn = n.din[l];
-    g.sbk = 1;
+    g.ldb = n.din[l];
     g.bias = n.P + n.boff[l];
     g.ldc = n.dout[l];
     if (l + 1 < n.L) {
-      g.pre = b.prel ? (*b.prel)[l] : b.pre;
+      g.pre = b.prel ? (*b.prel)[l] : nullptr;
       g.outb = b.hl ? (*b.hl)[l] : b.h[l % 2];
-      gemm<false, false, EPI_BIAS_ACT>(n, g);
+      gemm<EPI_BIAS_ACT>(n, g);
       a = g.outb;
     } else {
       g.outf = b.y;
-      gemm<false, false, EPI_BIAS>(n, g);
+      g.mrows = b.m;
+      gemm<EPI_BIAS>(n, g);
     }
   }
 }
 
-void forward(Net& n, int rows) {
+// forward pass of `rows` rows in n.x (or rows idx[r] of the resident set); output in n.y
+void forward(Net& n, int rows, const int* idx = nullptr) {
   Pass b{};
-  b.x = n.x;
+  b.x = idx ? n.X : n.x;
+  b.m = rows;
+  b.idx = idx;
   b.z = n.z;
   b.hl = &n.h;
   b.prel = &n.pre;
@@ -413,48 +588,49 @@ void forward(Net& n, int rows) {
   forward(n, rows, b);
 }
 
-// loss and gradients of the rows in (n.x, n.t, n.w); loss_row filled; gradients in n.G
-void backward(Net& n, int rows) {
+// loss and gradients of the rows in (n.x, n.t, n.w) or of rows idx[r] of the resident set;
+// loss_row filled; gradients in n.G
+void backward(Net& n, int rows, const int* idx = nullptr) {
   const int No = n.cfg.out_dim;
-  hipLaunchKernelGGL(k_loss, dim3(rows), dim3(256), 0, n.s, No, n.y, n.t, n.w, n.dA, n.loss_row);
+  hipLaunchKernelGGL(k_loss, dim3(rows), dim3(256), 0, n.s, No, n.y, idx ? n.T : n.t, idx ? n.W : n.w, idx, n.dA,
+                     n.loss_row);
   DGS_HIP(hipGetLastError());
   uint16_t* d = n.dA;  // gradient of layer l's pre-activation, [rows][dout[l]]
   uint16_t* d2 = n.dB;
   for (int l = n.L - 1; l >= 0; --l) {
-    const uint16_t* xin = l ? n.h[l - 1] : n.z;
     // dW_l = d^T xin
-    GemmArgs g{};
-    g.M = n.dout[l];
-    g.N = n.din[l];
-    g.K = rows;
-    g.A = d;
-    g.sam = 1;
-    g.sak = n.dout[l];
-    g.B = xin;
-    g.sbn = 1;
-    g.sbk = n.din[l];
-    g.outf = n.G + n.woff[l];
-    g.ldc = n.din[l];
-    gemm<true, true, EPI_STORE>(n, g);
-    hipLaunchKernelGGL(k_colsum, dim3((n.dout[l] + 255) / 256), dim3(256), 0, n.s, rows, n.dout[l], d,
+    GemmArgs w{};
+    w.M = w.mrows = n.dout[l];
+    w.N = n.din[l];
+    w.K = rows;
+    w.A = d;
+    w.lda = n.dout[l];
+    w.B = l ? n.h[l - 1] : n.z;
+    w.ldb = n.din[l];
+    w.outf = n.G + n.woff[l];
+    w.ldc = n.din[l];
+    check_gemm(w);
+    const int nw = (w.M / kSmall) * (w.N / kSmall);
+    // d_{l-1} = (d W_l) * silu'(pre_{l-1})
+    GemmArgs x{};
+    int nx = 0;
+    if (l) {
+      x.M = x.mrows = rows;
+      x.N = n.din[l];
+      x.K = n.dout[l];
+      x.A = d;
+      x.lda = n.dout[l];
+      x.B = n.Pb + n.woff[l];
+      x.ldb = n.din[l];
+      x.pre = n.pre[l - 1];
+      x.outb = d2;
+      x.ldc = n.din[l];
+      check_gemm(x);
+      nx = (x.M / kSmall) * (x.N / kSmall);
+    }
+    hipLaunchKernelGGL(k_backward, dim3(nx + nw + n.dout[l] / kSumCols), dim3(256), 0, n.s, x, nx, w, nw, rows,
                        n.G + n.boff[l]);
     DGS_HIP(hipGetLastError());
-    if (l == 0) break;
-    // d_{l-1} = (d W_l) * silu'(pre_{l-1})
-    GemmArgs b{};
-    b.M = rows;
-    b.N = n.din[l];
-    b.K = n.dout[l];
-    b.A = d;
-    b.sam = n.dout[l];
-    b.sak = 1;
-    b.B = n.Pb + n.woff[l];
-    b.sbn = 1;
-    b.sbk = n.din[l];
-    b.pre = n.pre[l - 1];
-    b.outb = d2;
-    b.ldc = n.din[l];
-    gemm<false, true, EPI_DACT>(n, b);
     std::swap(d, d2);
   }
 }
@@ -610,22 +786,19 @@ dgs_status dgs_forward_noalloc(dgs_net* n, int rows, const float* x, float* y) {
   return dgs::guarded(n, [&] {
     const int in = n->cfg.in_dim, No = n->cfg.out_dim;
     dgs::Pass b{};
-    // rows per pass: the largest multiple of 64 (up to max_batch) whose buffers fit the scratch array
-    int mb = 0;
-    for (int r = 64; r <= n->cfg.max_batch; r += 64)
-      if (dgs::scratch_layout(*n, r, nullptr, &b) <= dgs::kScratchBytes) mb = r;
-    if (!mb)
+    if (!dgs::scratch_takes(*n))
       throw dgs::Error(DGS_ERR_INVALID, "network too wide for the 16 MiB forward scratch (64 rows do not fit)");
+    // rows per pass: the largest multiple of 64 whose buffers fit the scratch array
+    int mb = 64 * (int)(dgs::kScratchBytes / dgs::scratch_layout(*n, 64, nullptr, nullptr));
     unsigned char* base = dgs::scratch_base(n->device);
     for (int r0 = 0; r0 < rows; r0 += mb) {
       const int m = std::min(mb, rows - r0);
       const int mp = (m + 63) / 64 * 64;  // whole 64-row tiles, padded with copies of the last row
       dgs::scratch_layout(*n, mp, base, &b);
-      hipLaunchKernelGGL(dgs::k_pad_rows, dim3((unsigned)((mp * in + 255) / 256)), dim3(256), 0, n->s,
-                         x + (size_t)r0 * in, m, mp, in, (float*)b.x);
-      DGS_HIP(hipGetLastError());
+      b.x = x + (size_t)r0 * in;
+      b.m = m;
+      b.y = y + (size_t)r0 * No;
       dgs::forward(*n, mp, b);
-      DGS_HIP(hipMemcpyAsync(y + (size_t)r0 * No, b.y, (size_t)m * No * sizeof(float), hipMemcpyDeviceToDevice, n->s));
     }
     DGS_HIP(hipStreamSynchronize(n->s));
   });
@@ -716,11 +889,9 @@ dgs_status dgs_train(dgs_net* n, int steps, int batch, float lr, uint64_t seed, 
       DGS_HIP(hipMemcpyAsync(didx, idx.data(), idx.size() * sizeof(int), hipMemcpyHostToDevice, n->s));
       const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
       for (int it = 0; it < steps; ++it) {
-        hipLaunchKernelGGL(dgs::k_gather, dim3(batch), dim3(256), 0, n->s, batch, n->cfg.in_dim, n->cfg.out_dim,
-                           didx + (size_t)it * batch, n->X, n->T, n->W, n->x, n->t, n->w);
-        DGS_HIP(hipGetLastError());
-        dgs::forward(*n, batch);
-        dgs::backward(*n, batch);
+        const int* bi = didx + (size_t)it * batch;
+        dgs::forward(*n, batch, bi);
+        dgs::backward(*n, batch, bi);
         hipLaunchKernelGGL(dgs::k_sum, dim3(1), dim3(256), 0, n->s, batch, n->loss_row, dloss + it);
         ++n->adam_t;
         const float c1 = 1.0f - std::pow(b1, (float)n->adam_t), c2 = 1.0f - std::pow(b2, (float)n->adam_t);

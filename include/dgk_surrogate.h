@@ -47,8 +47,8 @@ dgs_status dgs_forward(dgs_net* net, int rows, const float* x, float* y);
  * No counterpart in the reference. For callers that cannot allocate device memory (code under
  * HIP graph capture, tight serving loops): it calls no allocating routine; its activations live
  * in a fixed 16 MiB device array per GPU (rows are processed in passes of the largest multiple
- * of 64 whose buffers fit; a network whose 64-row pass does not fit is rejected with
- * DGS_ERR_INVALID). Ordered on the network's stream and synchronous like dgs_forward. Calls
+ * of 64 whose activations fit; a network of which 64 rows of inputs, activations and outputs do not
+ * fit is rejected with DGS_ERR_INVALID). Ordered on the network's stream and synchronous like dgs_forward. Calls
  * that overlap on one GPU share that array and race. */
 dgs_status dgs_forward_noalloc(dgs_net* net, int rows, const float* x, float* y);
 /* average device time of `reps` forward passes over `rows` rows already on the device */
