@@ -87,23 +87,33 @@ struct GemmArgs {
 // host), operands 16-byte aligned with lda and ldb multiples of 64.
 __device__ __forceinline__ f32x4 mma(const uint16_t* a, const uint16_t* b, f32x4 c) {
   const bf16x8 va = __builtin_bit_cast(bf16x8, *(const u32x4*)a), vb = __builtin_bit_cast(bf16x8, *(const u32x4*)b);
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(va, vb, c, 0, 0, 0);
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(vb, va, c, 0, 0, 0);
 }
 
+// The B fragment goes in as the matrix core's row operand, so that a lane's four results are four
+// consecutive columns of one row of C: one 8- or 16-byte access instead of four scattered ones.
+typedef float f32x4a4 __attribute__((ext_vector_type(4), aligned(4)));  // caller's memory: 4-byte aligned
 template <int EPI>
-__device__ __forceinline__ void gemm_store(const GemmArgs& g, int row, int col, float v) {
+__device__ __forceinline__ void gemm_store(const GemmArgs& g, int row, int col, f32x4 v) {
   if (row >= g.mrows || col >= g.N) return;
   const int64_t o = (int64_t)row * g.ldc + col;
   if (EPI == EPI_STORE) {
-    g.outf[o] = v;
-  } else if (EPI == EPI_BIAS_ACT) {
-    const float p = v + g.bias[col];
-    if (g.pre) g.pre[o] = p;
-    g.outb[o] = f2bf(silu(p));
+    *(f32x4*)(g.outf + o) = v;
   } else if (EPI == EPI_BIAS) {
-    g.outf[o] = v + g.bias[col];
+    *(f32x4a4*)(g.outf + o) = v + *(const f32x4*)(g.bias + col);
   } else {
-    g.outb[o] = f2bf(v * dsilu(g.pre[o]));
+    float r[4];
+    if (EPI == EPI_BIAS_ACT) {
+      const f32x4 p = v + *(const f32x4*)(g.bias + col);
+      if (g.pre) *(f32x4*)(g.pre + o) = p;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) r[i] = silu(p[i]);
+    } else {
+      const f32x4 p = *(const f32x4*)(g.pre + o);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) r[i] = v[i] * dsilu(p[i]);
+    }
+    *(u32x2*)(g.outb + o) = u32x2{f2bf(r[0]) | (uint32_t)f2bf(r[1]) << 16, f2bf(r[2]) | (uint32_t)f2bf(r[3]) << 16};
   }
 }
 
@@ -111,7 +121,7 @@ __device__ __forceinline__ void gemm_store(const GemmArgs& g, int row, int col, 
 // few hundred rows has only tens of 64x64 tiles for 256 CUs and is bound by memory latency, so the
 // tile is small and K goes through LDS in chunks of 256 (or its remainder, a multiple of 64), the next
 // two chunks' global loads in flight: one or two round trips cover a layer. 256 x 512 x 512: 10.1 ->
-// 4.6 us forward against 64x64 tiles loaded 32 k at a time without prefetch.
+// 4.1 us forward against 64x64 tiles loaded 32 k at a time without prefetch.
 // AT / BT: the operand is m- / n-contiguous in memory; a thread then loads 8 k-rows of 4 values and
 // transposes them in registers.
 constexpr int kSmall = 32, kChunk = 256, kSmallLd = kChunk + 8;
@@ -194,9 +204,7 @@ __device__ __forceinline__ void gemm_small(const GemmArgs& g, int bx, int by, ui
     chunk(k0, ra[0], rb[0]);
     chunk(k0 + kChunk, ra[1], rb[1]);
   }
-#pragma unroll
-  for (int r = 0; r < 4; ++r)
-    gemm_store<EPI>(g, m0 + wr + 4 * (lane >> 4) + r, n0 + wc + (lane & 15), acc[r]);
+  gemm_store<EPI>(g, m0 + wr + (lane & 15), n0 + wc + 4 * (lane >> 4), acc);
 }
 
 template <bool AT, bool BT, int EPI>
@@ -261,7 +269,7 @@ __global__ __launch_bounds__(256) void k_gemm_large(GemmArgs g) {
       for (int i = 0; i < F; ++i)
 #pragma unroll
         for (int j = 0; j < F; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[j], a[i], acc[i][j], 0, 0, 0);
     }
     if (k0 + 64 < g.K) store(buf ^ 1);
     __syncthreads();
@@ -270,9 +278,7 @@ __global__ __launch_bounds__(256) void k_gemm_large(GemmArgs g) {
   for (int i = 0; i < F; ++i)
 #pragma unroll
     for (int j = 0; j < F; ++j)
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        gemm_store<EPI>(g, m0 + wr + 16 * i + 4 * (lane >> 4) + r, n0 + wc + 16 * j + (lane & 15), acc[i][j][r]);
+      gemm_store<EPI>(g, m0 + wr + 16 * i + (lane & 15), n0 + wc + 16 * j + 4 * (lane >> 4), acc[i][j]);
 }
 
 // z[r][f] = sin(2 pi B_f . x_r), z[r][F + f] = cos(2 pi B_f . x_r), rounded to BF16.
@@ -302,6 +308,7 @@ __global__ __launch_bounds__(256) void k_loss(int N, const float* __restrict__ y
   const int64_t tr = idx ? idx[r] : r;
   const float wr = idx ? w[tr] / (float)(int)gridDim.x : w[tr];
   float s = 0;
+#pragma unroll 8
   for (int j = threadIdx.x; j < N; j += 256) {
     const int64_t o = (int64_t)r * N + j;
     const float d = y[o] - t[tr * N + j];
@@ -348,18 +355,19 @@ __device__ __forceinline__ void colsum(int M, int N, const uint16_t* __restrict_
 
 // Backward pass of one layer in one launch: the workgroups take the tiles of dX = (d W) silu'(pre)
 // (nx of them, none for the first layer), of dW = d^T x, and the bias gradient's column groups.
-__global__ __launch_bounds__(256) void k_backward(GemmArgs dx, int nx, GemmArgs dw, int nw, int rows, float* db) {
+__global__ __launch_bounds__(256) void k_backward(GemmArgs dx, int nx, GemmArgs dw, int rows, float* db) {
   __shared__ __attribute__((aligned(16))) uint16_t sh[2 * kSmall * kSmallLd];
   static_assert(2 * kSmall * kSmallLd >= kSumRows * kSumCols, "the column sums share the tiles' LDS");
   const int b = blockIdx.x;
-  if (b < nx) {
-    const int cols = dx.N / kSmall;
-    gemm_small<false, true, EPI_DACT>(dx, b % cols, b / cols, sh, sh + kSmall * kSmallLd);
-  } else if (b < nx + nw) {
-    const int t = b - nx, cols = dw.N / kSmall;
-    gemm_small<true, true, EPI_STORE>(dw, t % cols, t / cols, sh, sh + kSmall * kSmallLd);
+  const int ns = dw.M / kSumCols;  // the serial sums start first
+  if (b < ns) {
+    colsum(rows, dw.M, dw.A, db, b * kSumCols, sh);
+  } else if (b < ns + nx) {
+    const int t = b - ns, cols = dx.N / kSmall;
+    gemm_small<false, true, EPI_DACT>(dx, t % cols, t / cols, sh, sh + kSmall * kSmallLd);
   } else {
-    colsum(rows, dw.M, dw.A, db, (b - nx - nw) * kSumCols, sh);
+    const int t = b - ns - nx, cols = dw.N / kSmall;
+    gemm_small<true, true, EPI_STORE>(dw, t % cols, t / cols, sh, sh + kSmall * kSmallLd);
   }
 }
 
@@ -377,19 +385,27 @@ __global__ __launch_bounds__(256) void k_sum(int n, const float* __restrict__ v,
   if (threadIdx.x == 0) out[0] = red[0];
 }
 
-// Adam with bias correction; refreshes the BF16 copy of the weights.
-__global__ void k_adam(int64_t n, float* __restrict__ p, uint16_t* __restrict__ pb, const float* __restrict__ g,
-                       float* __restrict__ m, float* __restrict__ v, float lr, float b1, float b2, float c1, float c2,
+// Adam with bias correction; refreshes the BF16 copy of the weights. Four parameters per thread (the
+// parameter count is a multiple of 64).
+__global__ void k_adam(int64_t n4, f32x4* __restrict__ p, u32x2* __restrict__ pb, const f32x4* __restrict__ g,
+                       f32x4* __restrict__ m, f32x4* __restrict__ v, float lr, float b1, float b2, float c1, float c2,
                        float eps) {
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-    const float gi = g[i];
-    const float mi = b1 * m[i] + (1 - b1) * gi;
-    const float vi = b2 * v[i] + (1 - b2) * gi * gi;
+  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n4; i += (int64_t)gridDim.x * blockDim.x) {
+    const f32x4 gi = g[i];
+    f32x4 mi = m[i], vi = v[i], w = p[i];
+    uint32_t h[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      // one fixed order of rounding, whatever the compiler would contract
+      mi[k] = fmaf(1 - b1, gi[k], b1 * mi[k]);
+      vi[k] = fmaf(gi[k], (1 - b2) * gi[k], b2 * vi[k]);
+      w[k] = w[k] - lr * (mi[k] / c1) / (sqrtf(vi[k] / c2) + eps);
+      h[k] = f2bf(w[k]);
+    }
     m[i] = mi;
     v[i] = vi;
-    const float w = p[i] - lr * (mi / c1) / (sqrtf(vi / c2) + eps);
     p[i] = w;
-    pb[i] = f2bf(w);
+    pb[i] = u32x2{h[0] | h[1] << 16, h[2] | h[3] << 16};
   }
 }
 
@@ -466,14 +482,16 @@ void check_gemm(const GemmArgs& g) {
     throw Error(DGS_ERR_INVALID, "GEMM shape must be multiples of 64");
 }
 
-// C = A B with both operands k-contiguous (the forward pass): the largest tile whose grid still
-// fills the chip.
+// C = A B with both operands k-contiguous (the forward pass): the largest tile of which there are
+// enough for two or more workgroups per CU, since one alone waits for memory at every K step
+// (6528 x 512 x 512: 204 tiles of 128 take 25.9 us, 816 of 64 14.0 us; 6528 x 2048 x 512: 816 of 128
+// 34 us).
 template <int EPI>
 void gemm(Net& n, GemmArgs g) {
   check_gemm(g);
   auto grid = [&](int t) { return dim3((g.N + t - 1) / t, (g.M + t - 1) / t); };
   auto tiles = [&](int t) { return (int64_t)grid(t).x * grid(t).y; };
-  if (tiles(128) >= 192) hipLaunchKernelGGL((k_gemm_large<128, EPI>), grid(128), dim3(256), 0, n.s, g);
+  if (tiles(128) >= 512) hipLaunchKernelGGL((k_gemm_large<128, EPI>), grid(128), dim3(256), 0, n.s, g);
   else if (tiles(64) >= 384) hipLaunchKernelGGL((k_gemm_large<64, EPI>), grid(64), dim3(256), 0, n.s, g);
   else hipLaunchKernelGGL((k_gemm_small<false, false, EPI>), grid(kSmall), dim3(256), 0, n.s, g);
   DGS_HIP(hipGetLastError());
@@ -628,7 +646,7 @@ void backward(Net& n, int rows, const int* idx = nullptr) {
       check_gemm(x);
       nx = (x.M / kSmall) * (x.N / kSmall);
     }
-    hipLaunchKernelGGL(k_backward, dim3(nx + nw + n.dout[l] / kSumCols), dim3(256), 0, n.s, x, nx, w, nw, rows,
+    hipLaunchKernelGGL(k_backward, dim3(nx + nw + n.dout[l] / kSumCols), dim3(256), 0, n.s, x, nx, w, rows,
                        n.G + n.boff[l]);
     DGS_HIP(hipGetLastError());
     std::swap(d, d2);
@@ -895,8 +913,9 @@ dgs_status dgs_train(dgs_net* n, int steps, int batch, float lr, uint64_t seed, 
         hipLaunchKernelGGL(dgs::k_sum, dim3(1), dim3(256), 0, n->s, batch, n->loss_row, dloss + it);
         ++n->adam_t;
         const float c1 = 1.0f - std::pow(b1, (float)n->adam_t), c2 = 1.0f - std::pow(b2, (float)n->adam_t);
-        hipLaunchKernelGGL(dgs::k_adam, dim3(1024), dim3(256), 0, n->s, n->nparam, n->P, n->Pb, n->G, n->Am, n->Av,
-                           lr, b1, b2, c1, c2, eps);
+        hipLaunchKernelGGL(dgs::k_adam, dim3(2048), dim3(256), 0, n->s, n->nparam / 4, (dgs::f32x4*)n->P,
+                           (dgs::u32x2*)n->Pb, (const dgs::f32x4*)n->G, (dgs::f32x4*)n->Am, (dgs::f32x4*)n->Av, lr, b1,
+                           b2, c1, c2, eps);
         DGS_HIP(hipGetLastError());
       }
       if (losses) DGS_HIP(hipMemcpyAsync(losses, dloss, steps * sizeof(float), hipMemcpyDeviceToHost, n->s));
