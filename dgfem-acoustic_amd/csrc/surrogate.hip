@@ -222,7 +222,11 @@ __global__ __launch_bounds__(256) void k_gemm_large(GemmArgs g) {
   constexpr int LD = 72, W = BT / 2, F = W / 16, NL = BT / 32;
   __shared__ __attribute__((aligned(16))) uint16_t sA[2][BT * LD], sB[2][BT * LD];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int m0 = blockIdx.y * BT, n0 = blockIdx.x * BT;
+  // workgroup b runs on XCD b % 8: all column tiles of a row panel go to one XCD, whose L2 then
+  // fetches the panel once instead of all eight
+  const int cols = (g.N + BT - 1) / BT, t = blockIdx.x / 8;
+  const int m0 = (t / cols * 8 + blockIdx.x % 8) * BT, n0 = t % cols * BT;
+  if (m0 >= g.M) return;
   const int wr = (wave >> 1) * W, wc = (wave & 1) * W;
   f32x4 acc[F][F];
 #pragma unroll
@@ -489,11 +493,14 @@ void check_gemm(const GemmArgs& g) {
 template <int EPI>
 void gemm(Net& n, GemmArgs g) {
   check_gemm(g);
-  auto grid = [&](int t) { return dim3((g.N + t - 1) / t, (g.M + t - 1) / t); };
-  auto tiles = [&](int t) { return (int64_t)grid(t).x * grid(t).y; };
+  auto rows = [&](int t) { return (g.M + t - 1) / t; };
+  auto cols = [&](int t) { return (g.N + t - 1) / t; };
+  auto tiles = [&](int t) { return (int64_t)rows(t) * cols(t); };
+  auto grid = [&](int t) { return dim3((rows(t) + 7) / 8 * 8 * cols(t)); };  // row panels in eights, one per XCD
   if (tiles(128) >= 512) hipLaunchKernelGGL((k_gemm_large<128, EPI>), grid(128), dim3(256), 0, n.s, g);
   else if (tiles(64) >= 384) hipLaunchKernelGGL((k_gemm_large<64, EPI>), grid(64), dim3(256), 0, n.s, g);
-  else hipLaunchKernelGGL((k_gemm_small<false, false, EPI>), grid(kSmall), dim3(256), 0, n.s, g);
+  else
+    hipLaunchKernelGGL((k_gemm_small<false, false, EPI>), dim3(cols(kSmall), rows(kSmall)), dim3(256), 0, n.s, g);
   DGS_HIP(hipGetLastError());
 }
 
