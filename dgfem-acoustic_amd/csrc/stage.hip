@@ -347,6 +347,8 @@ struct MfmaLaunch {
   static constexpr int KB = 64 * WAVES;              // threads per workgroup
   static constexpr int TE = ROWSPLIT ? WAVES : 4 * WAVES;  // elements per tile (row split: 4 row groups)
   static constexpr int RG = WAVES / (TE / 4);        // row groups: waves sharing one element group
+  // waves that share their elements' work (k_stage_mfma): the workgroup in 2D FP32, one elsewhere
+  static constexpr int GW = RG == 1 && sizeof(T) == 4 && D == 2 ? WAVES : 1;
 };
 
 // Pad (in values) of the LDS element stride NP*ES. A wave's 4 elements read and write node rows at
@@ -413,8 +415,9 @@ struct MfmaCfg {
   static constexpr int PADV = lds_pad<T, ES>(NP);
   static constexpr int LES = NP * ES + PADV;
   // face fluxes [element][field][RBP], then the results in the state tile's layout
-  static constexpr int RBP = rb_stride<T>(M::RB);
-  static constexpr int NSB = 4 * TE * RBP > TE * LES ? 4 * TE * RBP : TE * LES;
+  static constexpr int RBP = rb_stride<T>(M::RB > (LES + 3) / 4 ? M::RB : (LES + 3) / 4);
+  static constexpr int NSB = 4 * TE * RBP;
+  static_assert(LES <= 4 * RBP, "an element's results take the place of its face fluxes");
   static constexpr size_t kLdsRest = sizeof(T) * (TE * LES + NSB + TE * NF * 4 + TE * 9) +
                                      sizeof(int) * NF * NPERM * NFP + (LO ? 16 * M::MB * M::NLO * 64 : 0);
   static constexpr size_t kLdsMax = 160 * 1024 - 512;
@@ -451,12 +454,24 @@ __global__ __launch_bounds__((MfmaLaunch<T, D, P, SH>::KB), (MfmaLaunch<T, D, P,
   constexpr int NCH = (RG > 1 && MBW == 1) ? 2 : 1;
   constexpr int VW = 16 / sizeof(T);                        // values per 16-byte vector
   typedef T VT __attribute__((ext_vector_type(VW)));
-  constexpr int PV = TE * NP / VW;                          // vectors per field of a tile (ES*PV in all)
-  // The state is node-interleaved, [element][node][field] with the ES live fields (nq), so a tile
-  // is one contiguous block of ES*PV vectors, a neighbour trace one load of ES values and a node's
+  // The GT threads of a group own GE elements of the tile and do all of their work: loads, face
+  // fluxes, contraction, time update. A group is GW waves (RG times as many in the row split). Groups
+  // share only the operator, so a group that is one wave meets no workgroup barrier in the tile loop,
+  // and the waves of a CU spread over the phases by themselves instead of computing, then waiting,
+  // together (five barriers a tile). us per stage (event-timed), workgroup -> wave: FP32 3D order 5,
+  // 82,944 elements, 151.6 -> 138.2; FP64 3D order 4, 48,000, 79.1 -> 72.0; FP64 2D order 2, 500,000,
+  // 87.5 -> 85.3; FP32 3D orders 3 and 4 unchanged. 2D FP32, where a wave's 4 elements leave most
+  // lanes of its loads idle, loses 2-3% and keeps the workgroup.
+  constexpr int GW = MfmaLaunch<T, D, P, SH>::GW, GT = 64 * RG * GW, GE = 4 * GW;
+  constexpr int GV = GE * NP * ES / VW;                     // 16-byte vectors of a group's state
+  // The state is node-interleaved, [element][node][field] with the ES live fields (nq), so a group's
+  // state is one contiguous block of GV vectors, a neighbour trace one load of ES values and a node's
   // fields one LDS read; the LDS tiles use the same layout.
   static_assert(ES == D + 1 || ES == 4, "ES: the live field count");
-  constexpr int NE = (4 * PV + kBlock - 1) / kBlock;        // state vectors per thread
+  static_assert(GE * NP * ES % VW == 0, "whole vectors per group");
+  constexpr int NE = (GV + GT - 1) / GT;                    // state vectors per thread
+  constexpr int NGEO = (GE * 9 + GT - 1) / GT;              // geometry values per thread
+  constexpr int NFC = (GE * NF * 4 + GT - 1) / GT;          // face geometry values per thread
   // Face work: TPF threads share one element face, thread kk of them taking the face nodes kk,
   // kk + TPF, ... (NI rounds), so that the face's connectivity, normal and flux coefficients are
   // loaded and formed once per thread and tile, every LDS address is an invariant of the thread plus
@@ -465,10 +480,8 @@ __global__ __launch_bounds__((MfmaLaunch<T, D, P, SH>::KB), (MfmaLaunch<T, D, P,
   // when every face node looked up its own face); us per stage before -> after: 3D order 3, 196,608
   // elements, FP32 85.1 -> 73.2, FP64 146 -> 124; 3D order 4, 115,000 elements, FP32 105 -> 94; 2D
   // order 2 FP64, 179,998 elements, 38.2 -> 34.6 (event-timed launches).
-  constexpr int TPF = kBlock / (TE * NF);
+  constexpr int TPF = GT / (GE * NF);
   constexpr int NI = (NFP + TPF - 1) / TPF;                 // face nodes per thread
-  constexpr int NGEO = (TE * 9 + kBlock - 1) / kBlock;      // geometry values per thread
-  constexpr int NFC = (TE * NF + kBlock - 1) / kBlock;      // element faces per thread
   typedef typename Mfma<T>::V V;
   constexpr int LES = C::LES;
   __shared__ __attribute__((aligned(32))) T sU[TE * LES];
@@ -476,19 +489,31 @@ __global__ __launch_bounds__((MfmaLaunch<T, D, P, SH>::KB), (MfmaLaunch<T, D, P,
   // sU's layout
   constexpr int NSB = C::NSB;
   __shared__ __attribute__((aligned(16))) T sB[NSB];
-  __shared__ T sN[TE * NF][4];
-  __shared__ T sG[TE][9];
+  __shared__ __attribute__((aligned(32))) T sN[TE * NF * 4];
+  __shared__ T sG[TE * 9];
   __shared__ uint32_t sVmap[NF * NPERM * NFP];  // byte offset of the neighbour's node in its element
   constexpr bool kALds = C::kALds;
   constexpr bool kCompact = C::kCompact;
   __shared__ T sA[kALds ? C::NAVS : 1];
   __shared__ bf16x8 sAlo[LO ? MB * NLO * 64 : 1];
-  T* const sR = sB;
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   // wave = rg * (TE/4) + element group; lane group g, column col = 4 * (element in group) + field q
   const int rg = RG > 1 ? wave / (TE / 4) : 0;
-  const int g = lane >> 4, col = lane & 15, el = (wave % (TE / 4)) * 4 + (col >> 2), q = col & 3;
+  const int we = wave % (TE / 4), grp = we / GW, gtid = (rg * GW + we % GW) * 64 + lane;
+  const int g = lane >> 4, col = lane & 15, el = we * 4 + (col >> 2), q = col & 3;
+  // a group's results take the place of its face fluxes, element el at el * LES of sR
+  T* const sR = sB + grp * GE * (4 * RB - LES);
+  // orders the group's LDS accesses: within one wave LDS works in program order and only the compiler
+  // has to keep it
+  auto sync = [&]() {
+    if constexpr (GT > 64) {
+      __syncthreads();
+    } else {
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+    }
+  };
   // 32-bit byte offsets: a buffer holds 4*PS*sizeof(T) < 2^32 bytes (checked at context creation)
   const T* __restrict__ Vin = (const T*)a.Vin;
   T* __restrict__ Vout = (T*)a.Vout;
@@ -522,21 +547,22 @@ __global__ __launch_bounds__((MfmaLaunch<T, D, P, SH>::KB), (MfmaLaunch<T, D, P,
 
   // Per-thread offsets that do not depend on the tile (every tile is full: the element count is
   // padded to a multiple of TE and padding elements carry zero state and geometry): the thread's
-  // state vectors sit at v*VW values into the tile, in a state buffer (add e0*NP*ES) and in LDS.
+  // state vectors sit at voff values into the tile in a state buffer (add e0*NP*ES), at loff in LDS.
   uint32_t voff[NE];
   int loff[NE];
 #pragma unroll
   for (int t = 0; t < NE; ++t) {
-    const int v = tid + t * kBlock;
-    voff[t] = (uint32_t)(v * VW);
-    loff[t] = v * VW + (v * VW / (NP * ES)) * C::PADV;
+    const int v = gtid + t * GT;
+    voff[t] = (uint32_t)(grp * GE * NP * ES + v * VW);
+    loff[t] = grp * GE * LES + v * VW + (v * VW / (NP * ES)) * C::PADV;
   }
+  auto has_vec = [&](int t) { return (t + 1) * GT <= GV || gtid + t * GT < GV; };
 
-  // The thread's element face and its nodes' places in the LDS state tile. Threads beyond the last
-  // face (2D: 16 of 256) repeat it without storing.
+  // The thread's element face and its nodes' places in the LDS state tile. Threads beyond the group's
+  // last face (2D: 4 of 64) repeat it without storing.
   static_assert(TPF >= 1, "every element face needs a thread");
-  const bool fact = TE * NF * TPF == kBlock || tid < TE * NF * TPF;
-  const int fp = fact ? tid / TPF : TE * NF - 1, kk = tid % TPF;
+  const bool fact = GE * NF * TPF == GT || gtid < GE * NF * TPF;
+  const int fp = grp * GE * NF + (fact ? gtid / TPF : GE * NF - 1), kk = gtid % TPF;
   const int fj = fp % NF;
   int fo[NI];
 #pragma unroll
@@ -550,7 +576,7 @@ __global__ __launch_bounds__((MfmaLaunch<T, D, P, SH>::KB), (MfmaLaunch<T, D, P,
   // and the (neighbour, code) pair of the thread's face are in flight into registers; the
   // neighbour traces of tile t+1 are gathered right after tile t's flux phase.
   VT pst[NE];
-  T pgeo[NGEO], pfg[NFC][4];
+  T pgeo[NGEO], pfg[NFC];
   int2 inc, cnc;
   T iqp[NI][4];
   // value `rel` of an array of `per` values per element, at the tile starting at element e0 (32-bit
@@ -563,19 +589,14 @@ __global__ __launch_bounds__((MfmaLaunch<T, D, P, SH>::KB), (MfmaLaunch<T, D, P,
   auto prefetch = [&](int64_t e0) {
 #pragma unroll
     for (int t = 0; t < NE; ++t)
-      if (tid + t * kBlock < nq * PV) pst[t] = *(const VT*)tile_at(Vin, e0, NP * ES, voff[t]);
+      if (has_vec(t)) pst[t] = *(const VT*)tile_at(Vin, e0, NP * ES, voff[t]);
 #pragma unroll
-    for (int t = 0; t < NGEO; ++t) {
-      const int idx = tid + t * kBlock;
-      if (idx < TE * 9) pgeo[t] = *tile_at(Jinv, e0, 9, (uint32_t)idx);
-    }
+    for (int t = 0; t < NGEO; ++t)
+      if (gtid + t * GT < GE * 9) pgeo[t] = *tile_at(Jinv, e0, 9, (uint32_t)(grp * GE * 9 + gtid + t * GT));
 #pragma unroll
-    for (int t = 0; t < NFC; ++t) {
-      const int idx = tid + t * kBlock;
-      if (idx < TE * NF)
-#pragma unroll
-        for (int c = 0; c < 4; ++c) pfg[t][c] = *tile_at(Fg, e0, NF * 4, (uint32_t)(idx * 4 + c));
-    }
+    for (int t = 0; t < NFC; ++t)
+      if (gtid + t * GT < GE * NF * 4)
+        pfg[t] = *tile_at(Fg, e0, NF * 4, (uint32_t)(grp * GE * NF * 4 + gtid + t * GT));
     inc = make_int2(*tile_at(a.nbr, e0, NF, (uint32_t)fp), *tile_at(a.code, e0, NF, (uint32_t)fp));
   };
   auto gather = [&]() {
@@ -604,23 +625,17 @@ __global__ __launch_bounds__((MfmaLaunch<T, D, P, SH>::KB), (MfmaLaunch<T, D, P,
   }
   for (int it = lb; valid(it); it += bpx) {
     const int64_t e0 = (int64_t)(xcd * tpx + it) * TE;
-    __syncthreads();  // the previous tile is done with LDS
+    sync();  // the previous tile is done with LDS
     // phase 1: commit the prefetched tile to LDS; epilogue operands and the next tile in flight
 #pragma unroll
     for (int t = 0; t < NE; ++t)
-      if (tid + t * kBlock < nq * PV) *(VT*)(sU + loff[t]) = pst[t];
+      if (has_vec(t)) *(VT*)(sU + loff[t]) = pst[t];
 #pragma unroll
-    for (int t = 0; t < NGEO; ++t) {
-      const int idx = tid + t * kBlock;
-      if (idx < TE * 9) sG[idx / 9][idx % 9] = pgeo[t];
-    }
+    for (int t = 0; t < NGEO; ++t)
+      if (gtid + t * GT < GE * 9) sG[grp * GE * 9 + gtid + t * GT] = pgeo[t];
 #pragma unroll
-    for (int t = 0; t < NFC; ++t) {
-      const int idx = tid + t * kBlock;
-      if (idx < TE * NF)
-#pragma unroll
-        for (int c = 0; c < 4; ++c) sN[idx][c] = pfg[t][c];
-    }
+    for (int t = 0; t < NFC; ++t)
+      if (gtid + t * GT < GE * NF * 4) sN[grp * GE * NF * 4 + gtid + t * GT] = pfg[t];
     // epilogue operands: issued here, a tile ahead of their use, when registers allow; shapes with
     // the operator in global memory load them just before the epilogue instead
     VT pu[NE], pa[NE];
@@ -639,7 +654,7 @@ __global__ __launch_bounds__((MfmaLaunch<T, D, P, SH>::KB), (MfmaLaunch<T, D, P,
     if (stage >= 1 && stage <= 3) {
 #pragma unroll
       for (int t = 0; t < NE; ++t)
-        if (tid + t * kBlock < nq * PV) {
+        if (has_vec(t)) {
           if (stage != 3 || CS) pu[t] = __builtin_nontemporal_load((const VT*)tile_at(U, e0, NP * ES, voff[t]));
           if (CS && stage == 3) plo[CS ? t : 0] = *(const uint2*)tile_at(Ulo, e0, NP * ES, voff[t]);
           if (CS || stage != 1)
@@ -655,7 +670,7 @@ __global__ __launch_bounds__((MfmaLaunch<T, D, P, SH>::KB), (MfmaLaunch<T, D, P,
     cnc = inc;
     const bool more = valid(it + bpx);
     if (more) prefetch((int64_t)(xcd * tpx + it + bpx) * TE);
-    __syncthreads();
+    sync();
     // phase 2: nodal normal numerical fluxes scaled by sJ/|detJ| -> sB[(e*4 + q)*RB + jk]. All three face
     // kinds share one form:
     //   fl = A (F(qm) + F(qp)).n-with-speed-vne + H (qm - qp),   F(q).n = (vne p + rc2 v.n, vne v + p/rho n)
@@ -669,8 +684,9 @@ __global__ __launch_bounds__((MfmaLaunch<T, D, P, SH>::KB), (MfmaLaunch<T, D, P,
     //   fs fl_p = fs A (vne (pm + pp) + rc2 (vm + vp).n) + fs H (pm - pp)
     //   fs fl_v = fs A (vne (vm + vp) + (pm + pp)/rho n) + fs H (vm - vp)
     {
-      const T n[3] = {sN[fp][0], sN[fp][1], sN[fp][2]};
-      const T fs = sN[fp][3];
+      T nf[4];
+      node_fields<4>(sN + fp * 4, nf);
+      const T n[3] = {nf[0], nf[1], nf[2]}, fs = nf[3];
       const bool inter = cnc.x >= 0, refl = cnc.x == -2;
       const T A = fs * ((inter || refl) ? (T)0.5 : (T)0.25);
       const T H = fs * (inter ? (T)0.5 * ((cnc.y >> 16) & 1 ? -c0 : c0) : (refl ? (T)0 : (T)0.25 * c0));
@@ -702,11 +718,11 @@ __global__ __launch_bounds__((MfmaLaunch<T, D, P, SH>::KB), (MfmaLaunch<T, D, P,
       }
     }
     if (more) gather();  // next tile's neighbour traces, in flight during the MFMA phase
-    __syncthreads();
+    sync();
     // phase 3: per-lane coefficients Ft_r = alpha_r p + sum_x beta_rx v_x, then the MFMA chain
     T alpha[D], beta[D][3];
     {
-      const T* G = sG[el];
+      const T* G = sG + el * 9;
       for (int r = 0; r < D; ++r) {
         const T at = G[r * 3 + 0] * v0[0] + G[r * 3 + 1] * v0[1] + G[r * 3 + 2] * v0[2];
         if (q == 0) {
@@ -786,7 +802,7 @@ __global__ __launch_bounds__((MfmaLaunch<T, D, P, SH>::KB), (MfmaLaunch<T, D, P,
     } else {
       chain(std::integral_constant<int, 64>{});
     }
-    __syncthreads();  // face fluxes consumed; sB now receives the results in the LDS tile's layout
+    sync();  // face fluxes consumed; their place receives the results in the LDS tile's layout
 #pragma unroll
     for (int mb = 0; mb < MBW; ++mb) {
       V r = acc[mb * NCH];
@@ -814,13 +830,13 @@ __global__ __launch_bounds__((MfmaLaunch<T, D, P, SH>::KB), (MfmaLaunch<T, D, P,
         if (i < NP && q < nq) sR[el * LES + i * ES + q] = (T)acct[t];
       }
     }
-    __syncthreads();
+    sync();
     if (kDefer && !kALds) load_epi();
     // phase 4: time-integration epilogue on 16-byte vectors
     const T s6 = (T)(1.0 / 6.0), s3 = (T)(1.0 / 3.0), s2 = (T)0.5;
 #pragma unroll
     for (int t = 0; t < NE; ++t) {
-      if (tid + t * kBlock >= nq * PV) break;
+      if (!has_vec(t)) break;
       const VT kq = dt * *(const VT*)(sR + loff[t]);
       VT* const pAcc = (VT*)tile_at(Acc, e0, NP * ES, voff[t]);
       VT* const pOut = (VT*)tile_at(Vout, e0, NP * ES, voff[t]);
