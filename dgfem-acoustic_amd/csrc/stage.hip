@@ -494,7 +494,7 @@ __global__ __launch_bounds__((MfmaLaunch<T, D, P, SH>::KB), (MfmaLaunch<T, D, P,
   __shared__ uint32_t sVmap[NF * NPERM * NFP];  // byte offset of the neighbour's node in its element
   constexpr bool kALds = C::kALds;
   constexpr bool kCompact = C::kCompact;
-  __shared__ T sA[kALds ? C::NAVS : 1];
+  __shared__ __attribute__((aligned(16))) T sA[kALds ? C::NAVS : 1];
   __shared__ bf16x8 sAlo[LO ? MB * NLO * 64 : 1];
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -528,23 +528,12 @@ __global__ __launch_bounds__((MfmaLaunch<T, D, P, SH>::KB), (MfmaLaunch<T, D, P,
   const T v0[3] = {(T)a.v0[0], (T)a.v0[1], (T)a.v0[2]};
   const int stage = a.stage;
   constexpr int nq = ES;  // the buffers hold exactly the live fields
-  for (int i = tid; i < NF * NPERM * NFP; i += kBlock) sVmap[i] = (uint32_t)a.vmap[i] * (uint32_t)(ES * sizeof(T));
-  if (kALds) {
-    constexpr int NFULL = kCompact ? (MBF - 1) * KS * 64 : NAV;
-    for (int i = tid; i < NFULL; i += kBlock) sA[i] = Af[i];
-    if constexpr (kCompact)  // the last block without its zero rows: value c of a k-step is row c%8, k c/8
-      for (int i = tid; i < KS * 32; i += kBlock)
-        sA[NFULL + i] = Af[NFULL + (i / 32) * 64 + ((i % 32) / 8) * 16 + (i % 8)];
-  }
   static_assert(RG == 1 || kALds, "row split keeps the operator in LDS");
   // the wave of the compact last block (wave-uniform)
   const bool clast = kCompact && rg == MBF - 1;
   const T* __restrict__ pA = clast ? (const T*)sA + (MBF - 1) * KS * 64 + (lane >> 4) * 8 + (lane & 7)
                                    : (kALds ? (const T*)sA : Af) + lane + rg * (MBW * KS * 64);
   const T* __restrict__ pT = (kALds ? (const T*)sA : Af) + MBF * KS * 64 + 4 * (lane >> 4) + (lane & 3);
-  if (LO)
-    for (int i = tid; i < MB * NLO * 64; i += kBlock) sAlo[i] = ((const bf16x8*)a.Alo)[i];
-
   // Per-thread offsets that do not depend on the tile (every tile is full: the element count is
   // padded to a multiple of TE and padding elements carry zero state and geometry): the thread's
   // state vectors sit at voff values into the tile in a state buffer (add e0*NP*ES), at loff in LDS.
@@ -618,11 +607,40 @@ __global__ __launch_bounds__((MfmaLaunch<T, D, P, SH>::KB), (MfmaLaunch<T, D, P,
   const int bpx = rr ? gridDim.x : gridDim.x / 8;
   const int tpx = rr ? (int)a.tiles : a.tiles_per_xcd, ntiles = (int)a.tiles;
   auto valid = [&](int it) { return it < tpx && xcd * tpx + it < ntiles; };
-  __syncthreads();  // sVmap ready for the first gathers
-  if (valid(lb)) {
-    prefetch((int64_t)(xcd * tpx + lb) * TE);
-    gather();
+  // Start: the first tile's loads, then the tables and the operator in batches of independent loads, so
+  // that a workgroup with one tile (small meshes) waits for one memory round trip before its gathers
+  // instead of one per 256 operator values (us per stage in graph replay: 2D order 3 FP64, 3200 elements,
+  // 4.11 -> 3.80; event-timed: 3D order 5 FP64, 7722 elements, whose operator is 110 KB, 41.0 -> 35.9).
+  const bool first = valid(lb);
+  if (first) prefetch((int64_t)(xcd * tpx + lb) * TE);
+#pragma unroll
+  for (int i = 0; i < NF * NPERM * NFP; i += kBlock)
+    if (i + tid < NF * NPERM * NFP) sVmap[i + tid] = (uint32_t)a.vmap[i + tid] * (uint32_t)(ES * sizeof(T));
+  if constexpr (kALds) {
+    // 16-byte vectors of the operator as LDS holds it; in the compact form the last block comes
+    // without its zero rows: value c of a k-step is row c%8 at k c/8
+    constexpr int NFULL = kCompact ? (MBF - 1) * KS * 64 : NAV, NV = C::NAVS / VW, NB = 8;
+    static_assert(NFULL % VW == 0 && C::NAVS % VW == 0 && 8 % VW == 0, "whole vectors");
+    auto src = [&](int v) {
+      const int i = v * VW;
+      if (!kCompact || i < NFULL) return i;
+      const int c = i - NFULL;
+      return NFULL + (c / 32) * 64 + ((c % 32) / 8) * 16 + c % 8;
+    };
+    for (int v0 = tid; v0 < NV; v0 += NB * kBlock) {
+      VT r[NB];
+#pragma unroll
+      for (int k = 0; k < NB; ++k)
+        if (v0 + k * kBlock < NV) r[k] = *(const VT*)(Af + src(v0 + k * kBlock));
+#pragma unroll
+      for (int k = 0; k < NB; ++k)
+        if (v0 + k * kBlock < NV) *(VT*)(sA + (v0 + k * kBlock) * VW) = r[k];
+    }
   }
+  if (LO)
+    for (int i = tid; i < MB * NLO * 64; i += kBlock) sAlo[i] = ((const bf16x8*)a.Alo)[i];
+  __syncthreads();  // the tables and the operator are in LDS
+  if (first) gather();
   for (int it = lb; valid(it); it += bpx) {
     const int64_t e0 = (int64_t)(xcd * tpx + it) * TE;
     sync();  // the previous tile is done with LDS
