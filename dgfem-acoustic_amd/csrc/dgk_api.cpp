@@ -385,7 +385,7 @@ StageArgs base_args(Ctx& c) {
 }
 
 // Launch the four RK4 stages of one step on stream s.
-void rk4_step(Ctx& c, double dt, hipStream_t s, hipEvent_t* ev) {
+void rk4_stages(Ctx& c, double dt, hipStream_t s, hipEvent_t* ev) {
   StageArgs a = base_args(c);
   a.dt = dt;
   void* in[4] = {c.U, c.V0, c.V1, c.V0};
@@ -398,7 +398,11 @@ void rk4_step(Ctx& c, double dt, hipStream_t s, hipEvent_t* ev) {
     launch_stage(c, a, s);
     if (ev) DGK_HIP(hipEventRecord(ev[2 * st + 1], s));
   }
-  launch_record(c, s);
+}
+
+void rk4_step(Ctx& c, double dt, hipStream_t s, hipEvent_t* ev) {
+  rk4_stages(c, dt, s, ev);
+  launch_edge(c, true, false, s);
 }
 
 namespace {
@@ -535,7 +539,7 @@ void install_receivers(Ctx& c, const std::vector<int64_t>& elem, const std::vect
   DGK_HIP(hipMalloc(&c.rec.base, n * sizeof(int64_t)));
   DGK_HIP(hipMalloc(&c.rec.w, (size_t)n * c.Np * c.tsize));
   DGK_HIP(hipMalloc(&c.rec.out, (size_t)n * cap * c.tsize));
-  DGK_HIP(hipMalloc(&c.rec.counter, sizeof(int)));
+  DGK_HIP(hipMalloc(&c.rec.counter, 2 * sizeof(int)));
   c.rec.n = n;
   c.rec.cap = cap;
   DGK_HIP(hipMemcpy(c.rec.base, base.data(), n * sizeof(int64_t), hipMemcpyHostToDevice));
@@ -545,7 +549,7 @@ void install_receivers(Ctx& c, const std::vector<int64_t>& elem, const std::vect
     std::vector<float> wf(w.begin(), w.end());
     DGK_HIP(hipMemcpy(c.rec.w, wf.data(), wf.size() * sizeof(float), hipMemcpyHostToDevice));
   }
-  DGK_HIP(hipMemset(c.rec.counter, 0, sizeof(int)));
+  DGK_HIP(hipMemset(c.rec.counter, 0, 2 * sizeof(int)));
 }
 
 // Put rows x rec.n host values back into a freshly installed record and continue after them.
@@ -602,12 +606,10 @@ hipGraphExec_t rk4_graph(Ctx& c, int steps, double dt, bool src) {
   hipGraph_t g;
   DGK_HIP(hipStreamBeginCapture(c.stream, hipStreamCaptureModeThreadLocal));
   try {
+    if (src) launch_edge(c, false, true, c.stream);
     for (int k = 0; k < steps; ++k) {
-      if (src) {
-        for (auto& s : c.sources) launch_source_timed(c, s, c.stream);
-        launch_tick(c, c.stream);
-      }
-      rk4_step(c, dt, c.stream);
+      rk4_stages(c, dt, c.stream);
+      launch_edge(c, true, src && k + 1 < steps, c.stream);
     }
   } catch (...) {
     hipGraph_t junk = nullptr;
@@ -665,7 +667,7 @@ void euler_impl(Ctx& c, int nsteps, double dt, const double* ts) {
     launch_stage(c, a, c.stream);
     std::swap(c.U, c.V0);  // graphs capture buffer addresses; drop any cached one
     c.drop_graphs();
-    launch_record(c, c.stream);
+    launch_edge(c, true, false, c.stream);
   }
 }
 

@@ -140,7 +140,7 @@ struct Ctx {
     int64_t* base = nullptr;  // [n] offset e*Np of the receiver's element in the pressure plane
     void* w = nullptr;       // [n][Np] basis weights in the state type
     void* out = nullptr;     // [cap][n] recorded pressure in the state type
-    int* counter = nullptr;  // rows recorded so far (device)
+    int* counter = nullptr;  // rows recorded so far, and k_edge's count of finished workgroups (device)
   } rec;
   void free_receivers();
   int64_t device_bytes = 0;
@@ -178,10 +178,9 @@ void launch_stage(Ctx& c, StageArgs& a, hipStream_t s);
 // fields, buffer sizes); `a` as for launch_stage, nothing is launched
 bool tile_shape_supported(Ctx& c, StageArgs& a, int shape);
 void launch_source(Ctx& c, const Ctx::Src& s, double value, hipStream_t st);
-// hard source overwrite at the step whose start time is c.tdev[*c.tstep] (when t < duration)
-void launch_source_timed(Ctx& c, const Ctx::Src& s, hipStream_t st);
-void launch_tick(Ctx& c, hipStream_t st);  // ++*c.tstep
-void launch_record(Ctx& c, hipStream_t st);  // no-op without receivers
+// the work between two steps: with `record`, record the receivers (if any); then, with `source`, the
+// hard source overwrite at the step whose start time is c.tdev[*c.tstep] (when t < duration) and ++*c.tstep
+void launch_edge(Ctx& c, bool record, bool source, hipStream_t st);
 bool check_finite(Ctx& c);
 // FP64 field planes on the device (plane stride PS; element nodes [off, off+n) of each plane) -> a
 // state buffer in the context's precision and layout; in the FP32 compensated form lo (if given)
@@ -194,7 +193,8 @@ void mfma_shape(int dim, int p, bool fp32, bool oplo, int* KS, int* MB, int* NT)
 // dgk_api.cpp
 extern thread_local std::string g_err;
 void create_impl(Ctx& c, const dgk_mesh* m, const dgk_phys* ph, const dgk_opts* o);
-void rk4_step(Ctx& c, double dt, hipStream_t s, hipEvent_t* ev = nullptr);
+void rk4_stages(Ctx& c, double dt, hipStream_t s, hipEvent_t* ev = nullptr);
+void rk4_step(Ctx& c, double dt, hipStream_t s, hipEvent_t* ev = nullptr);  // the stages and the record
 StageArgs base_args(Ctx& c);  // stage-kernel arguments over the context's buffers
 double* staging(Ctx& c);
 int live_planes(int dim, const double* u, int64_t n);  // nq of a host state u[4][n]

@@ -42,6 +42,21 @@ struct Sz {
 namespace {
 
 constexpr int kBlock = 256;
+constexpr int kEdgeBlock = 1024;
+
+// Sources of one k_edge launch (n = 0: none).
+struct EdgeArgs {
+  static constexpr int kMax = 8;
+  struct Source {
+    const int64_t* idx;
+    int64_t n;
+    double amp, freq, phase, duration;
+  };
+  int n;
+  const double* tdev;
+  int* tstep;
+  Source s[kMax];
+};
 
 template <typename T, int D, int P>
 __global__ __launch_bounds__(kBlock) void k_stage_lds(StageArgs a) {
@@ -945,32 +960,69 @@ __global__ void k_tick(int* __restrict__ tstep) {
   if (threadIdx.x == 0) *tstep += 1;
 }
 
-// One workgroup: every thread interpolates receivers r = tid, tid+256, ... from the pressure field
-// (value (e*Np + node)*es of the state buffer) and writes row *counter of the record; the row index is read before and advanced after the
-// writes, so a captured graph records consecutive rows on every replay. Rows beyond cap are dropped.
+__device__ __forceinline__ float lane_value(float v, int k) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), k));
+}
+__device__ __forceinline__ double lane_value(double v, int k) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), k),
+                          __builtin_amdgcn_readlane(__double2loint(v), k));
+}
+
+// The work between two time steps, in one launch: record the receivers of the step that ended, then
+// overwrite the sources' pressure for the step that begins (EdgeArgs, either part may be empty).
+// Record: a wave per receiver interpolates the pressure (value (e*Np + node)*es of the state buffer),
+// its lanes loading the nodes together, the sum taken in node order; row counter[0] of the record is
+// written and the last workgroup to finish advances the row (counter[1] counts them), so a captured
+// graph records consecutive rows on every replay. Rows beyond cap are dropped. A thread walking the
+// nodes of its receiver took a memory round trip every few nodes: 64 receivers at 3D order 4, 22.2 ->
+// 5.7 us.
+// Sources (one workgroup): the source values at the step whose start time is tdev[*tstep], one source
+// after the other as later ones win, then ++*tstep; separate launches for the record, each source and
+// the step count cost about 1.5-2.5 us each on a small mesh whose stages take 3.5 us.
 template <typename T>
-__global__ void k_record(const T* __restrict__ U, const uint16_t* __restrict__ Ulo, const int64_t* __restrict__ base,
-                         const T* __restrict__ w, int n, int Np, T* __restrict__ out, int* __restrict__ counter,
-                         int cap, int es) {
-  __shared__ int row;
-  if (threadIdx.x == 0) row = *counter;
-  __syncthreads();
-  const int r0 = row;
-  if (r0 < cap) {
-    for (int r = threadIdx.x; r < n; r += blockDim.x) {
-      const int64_t b = base[r];
-      T acc = 0;
-      for (int k = 0; k < Np; ++k) {
-        const int64_t j = (int64_t)(b + k) * es;  // pressure of node k
-        T u = U[j];
-        if (Ulo) u += (T)bf16_bits_to_f32(Ulo[j]);
-        acc += w[r * Np + k] * u;
+__global__ __launch_bounds__(kEdgeBlock) void k_edge(T* U, uint16_t* Ulo, int es, const int64_t* __restrict__ base,
+                                                     const T* __restrict__ w, int n, int Np, T* __restrict__ out,
+                                                     int* counter, int cap, EdgeArgs src) {
+  const int tid = threadIdx.x, lane = tid & 63;
+  const double t = src.n ? src.tdev[*src.tstep] : 0.0;
+  if (n) {
+    const int row = counter[0];
+    if (row < cap)
+      for (int r = (blockIdx.x * kEdgeBlock + tid) >> 6; r < n; r += (gridDim.x * kEdgeBlock) >> 6) {
+        T u = 0, c = 0;
+        if (lane < Np) {
+          const int64_t j = (base[r] + lane) * es;  // pressure of node `lane`
+          u = U[j];
+          if (Ulo) u += (T)bf16_bits_to_f32(Ulo[j]);
+          c = w[r * Np + lane];
+        }
+        T acc = 0;
+        for (int k = 0; k < Np; ++k) acc = fma(lane_value(c, k), lane_value(u, k), acc);
+        if (lane == 0) out[(int64_t)row * n + r] = acc;
       }
-      out[(int64_t)r0 * n + r] = acc;
+    __syncthreads();
+    if (tid == 0) {
+      __threadfence();
+      if (atomicAdd(counter + 1, 1) == (int)gridDim.x - 1) {
+        counter[1] = 0;
+        if (row < cap) counter[0] = row + 1;
+      }
     }
   }
-  __syncthreads();
-  if (threadIdx.x == 0 && r0 < cap) *counter = r0 + 1;
+  if (!src.n) return;
+  for (int s = 0; s < src.n; ++s) {
+    const EdgeArgs::Source& q = src.s[s];
+    if (t < q.duration) {
+      const T value = (T)(q.amp * sin(2 * M_PI * q.freq * t + q.phase));
+      for (int64_t i = tid; i < q.n; i += kEdgeBlock) {
+        const int64_t j = q.idx[i] * es;
+        U[j] = value;
+        if (Ulo) Ulo[j] = 0;
+      }
+    }
+    __syncthreads();
+  }
+  if (tid == 0) *src.tstep += 1;
 }
 
 template <typename T>
@@ -1203,36 +1255,64 @@ void launch_source(Ctx& c, const Ctx::Src& src, double value, hipStream_t st) {
   DGK_HIP(hipGetLastError());
 }
 
-void launch_source_timed(Ctx& c, const Ctx::Src& src, hipStream_t st) {
-  if (!src.n) return;
-  const unsigned nb = (unsigned)std::min<int64_t>((src.n + 255) / 256, 1024);
-  if (c.precision == DGK_FP64)
-    hipLaunchKernelGGL(k_source_timed<double>, dim3(nb), dim3(256), 0, st, (double*)c.U, (uint16_t*)nullptr, src.idx,
-                       src.n, src.amp, src.freq, src.phase, src.duration, (const double*)c.tdev,
-                       (const int*)c.tstep, c.es);
-  else
-    hipLaunchKernelGGL(k_source_timed<float>, dim3(nb), dim3(256), 0, st, (float*)c.U,
-                       (uint16_t*)(c.comp ? c.Ulo : nullptr), src.idx, src.n, src.amp, src.freq, src.phase,
-                       src.duration, (const double*)c.tdev, (const int*)c.tstep, c.es);
+namespace {
+
+// a single workgroup overwrites the sources between two steps while they are few and small
+constexpr int64_t kEdgeNodes = 8192;
+bool sources_fit_edge(const Ctx& c) {
+  int64_t n = 0;
+  for (auto& s : c.sources) n += s.n;
+  return c.sources.size() <= EdgeArgs::kMax && n <= kEdgeNodes;
+}
+
+template <typename T>
+void edge(Ctx& c, bool record, bool source, hipStream_t st) {
+  EdgeArgs e{};
+  if (source) {
+    for (auto& s : c.sources)
+      if (s.n) e.s[e.n++] = {s.idx, s.n, s.amp, s.freq, s.phase, s.duration};
+    e.tdev = c.tdev;
+    e.tstep = c.tstep;
+  }
+  const int n = record ? c.rec.n : 0;
+  // a wave per receiver, up to a workgroup per CU; the sources' order needs one workgroup
+  const int blocks = e.n ? 1 : std::min((n + kEdgeBlock / 64 - 1) / (kEdgeBlock / 64), 256);
+  hipLaunchKernelGGL(k_edge<T>, dim3(blocks), dim3(kEdgeBlock), 0, st, (T*)c.U,
+                     sizeof(T) == 4 && c.comp ? c.Ulo : nullptr, c.es, c.rec.base, (const T*)c.rec.w, n, c.Np,
+                     (T*)c.rec.out, c.rec.counter, c.rec.cap, e);
   DGK_HIP(hipGetLastError());
 }
 
-void launch_tick(Ctx& c, hipStream_t st) {
+template <typename T>
+void sources_timed(Ctx& c, hipStream_t st) {
+  for (auto& src : c.sources) {
+    if (!src.n) continue;
+    const unsigned nb = (unsigned)std::min<int64_t>((src.n + 255) / 256, 1024);
+    hipLaunchKernelGGL(k_source_timed<T>, dim3(nb), dim3(256), 0, st, (T*)c.U,
+                       sizeof(T) == 4 && c.comp ? c.Ulo : nullptr, src.idx, src.n, src.amp, src.freq, src.phase,
+                       src.duration, (const double*)c.tdev, (const int*)c.tstep, c.es);
+    DGK_HIP(hipGetLastError());
+  }
   hipLaunchKernelGGL(k_tick, dim3(1), dim3(64), 0, st, c.tstep);
   DGK_HIP(hipGetLastError());
 }
 
-void launch_record(Ctx& c, hipStream_t st) {
-  if (!c.rec.n) return;
-  if (c.precision == DGK_FP64)
-    hipLaunchKernelGGL(k_record<double>, dim3(1), dim3(256), 0, st, (const double*)c.U, (const uint16_t*)nullptr,
-                       c.rec.base, (const double*)c.rec.w, c.rec.n, c.Np, (double*)c.rec.out, c.rec.counter,
-                       c.rec.cap, c.es);
-  else
-    hipLaunchKernelGGL(k_record<float>, dim3(1), dim3(256), 0, st, (const float*)c.U,
-                       (const uint16_t*)(c.comp ? c.Ulo : nullptr), c.rec.base, (const float*)c.rec.w, c.rec.n,
-                       c.Np, (float*)c.rec.out, c.rec.counter, c.rec.cap, c.es);
-  DGK_HIP(hipGetLastError());
+}  // namespace
+
+void launch_edge(Ctx& c, bool record, bool source, hipStream_t st) {
+  record = record && c.rec.n;
+  if (!record && !source) return;
+  // many receivers keep a workgroup each to themselves
+  const bool fit = source && sources_fit_edge(c), together = fit && (!record || c.rec.n <= 4 * kEdgeBlock / 64);
+  auto run = [&](bool r, bool s) {
+    if (c.precision == DGK_FP64) edge<double>(c, r, s, st);
+    else edge<float>(c, r, s, st);
+  };
+  if (together || !source) return run(record, source);
+  if (record) run(true, false);
+  if (fit) run(false, true);
+  else if (c.precision == DGK_FP64) sources_timed<double>(c, st);
+  else sources_timed<float>(c, st);
 }
 
 bool check_finite(Ctx& c) {
