@@ -7,6 +7,7 @@
 #include <sstream>
 #include <cmath>
 #include <cstring>
+#include <exception>
 #include <unordered_map>
 
 #include "dgk_internal.hpp"
@@ -440,24 +441,105 @@ double bary_score(int d, int Np, const double* node_xyz, int64_t e, const double
 }  // namespace
 
 // Locate points xyz[n][3] in a mesh given by its element node coordinates (Gmsh order, vertices
-// first): for each point the element whose smallest barycentric coordinate of the point is
-// largest. Elements are binned by bounding box into a uniform grid of about K cells, so each
-// point tests only the elements of its cell. Returns the elements; w receives, per point, the
-// element's Lagrange basis at the point (pressure = sum_n w[n] p[e*Np + n]).
+// first): for each point, of the elements whose bounding box meets the point's cell in a uniform grid
+// of about K cells, the one whose smallest barycentric coordinate of the point is largest. Returns the
+// elements; w receives, per point, the element's Lagrange basis at the point (pressure = sum_n w[n]
+// p[e*Np+n]).
+// The points are binned, not the elements: one pass over the vertices on several threads finds the mesh's
+// extent and the few elements whose (slightly grown) box holds a point; an element that accepts a point
+// (coordinate >= -1e-6) is among them. 196,608 elements, 16 points: 24.4 -> 2.8 ms.
 std::vector<int64_t> locate_points(const RefElem& R, const double* node_xyz, int64_t K, int n, const double* xyz,
                                    std::vector<double>& w) {
   const int d = R.dim, Np = R.Np;
   std::vector<int64_t> out(n, -1);
   w.assign((size_t)n * Np, 0.0);
   if (!n) return out;
-  double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300};
-  for (int64_t e = 0; e < K; ++e)
-    for (int v = 0; v <= d; ++v)
+  // a uniform grid over the points' own extent, about one point a cell
+  double plo[3], phi_[3];
+  for (int c = 0; c < 3; ++c) {
+    plo[c] = 1e300;
+    phi_[c] = -1e300;
+    for (int p = 0; p < n; ++p) {
+      plo[c] = std::min(plo[c], xyz[3 * p + c]);
+      phi_[c] = std::max(phi_[c], xyz[3 * p + c]);
+    }
+  }
+  int pg[3] = {1, 1, 1};
+  const int pgd = (int)std::max(1.0, std::floor(std::pow((double)n, 1.0 / d)));
+  for (int c = 0; c < d; ++c) pg[c] = pgd;
+  auto pcell = [&](int c, double q) {
+    const double span = phi_[c] - plo[c], f = span > 0 ? (q - plo[c]) / span * pg[c] : 0;
+    return f > 0 ? (int)std::min(f, pg[c] - 1.0) : 0;
+  };
+  std::vector<int> pstart((size_t)pg[0] * pg[1] * pg[2] + 1, 0), pitem(n);
+  auto pindex = [&](int i, int j, int k) { return ((size_t)i * pg[1] + j) * pg[2] + k; };
+  auto pof = [&](int p) { return pindex(pcell(0, xyz[3 * p]), pcell(1, xyz[3 * p + 1]), pcell(2, xyz[3 * p + 2])); };
+  for (int p = 0; p < n; ++p) ++pstart[pof(p) + 1];
+  for (size_t i = 1; i < pstart.size(); ++i) pstart[i] += pstart[i - 1];
+  {
+    std::vector<int> fill(pstart.begin(), pstart.end() - 1);
+    for (int p = 0; p < n; ++p) pitem[fill[pof(p)]++] = p;
+  }
+  struct Hit {
+    int p;
+    int64_t e;
+  };
+  struct Found {
+    double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300};
+    std::vector<Hit> hits;
+    std::exception_ptr err;
+  };
+  auto bounds = [&](int64_t e, double a[3], double b[3]) {
+    const double* X = node_xyz + (size_t)e * Np * 3;
+    for (int c = 0; c < 3; ++c) a[c] = b[c] = X[c];
+    for (int v = 1; v <= d; ++v)
       for (int c = 0; c < 3; ++c) {
-        const double q = node_xyz[((size_t)e * Np + v) * 3 + c];
-        lo[c] = std::min(lo[c], q);
-        hi[c] = std::max(hi[c], q);
+        a[c] = std::min(a[c], X[3 * v + c]);
+        b[c] = std::max(b[c], X[3 * v + c]);
       }
+  };
+  std::vector<Found> found(8);
+  parallel_ranges(K, 16384, [&](int t, int64_t e0, int64_t e1) {
+    Found& f = found[t];
+    try {
+      for (int64_t e = e0; e < e1; ++e) {
+        double a[3], b[3];
+        bounds(e, a, b);
+        bool out_of_reach = false;
+        for (int c = 0; c < 3; ++c) {
+          f.lo[c] = std::min(f.lo[c], a[c]);
+          f.hi[c] = std::max(f.hi[c], b[c]);
+          if (c >= d) continue;
+          const double grow = 1e-4 * (b[c] - a[c]) + 1e-8 * (1 + std::fabs(a[c]) + std::fabs(b[c]));
+          a[c] -= grow;
+          b[c] += grow;
+          out_of_reach |= !(b[c] >= plo[c] && a[c] <= phi_[c]);
+        }
+        if (out_of_reach) continue;
+        for (int i = pcell(0, a[0]), i1 = pcell(0, b[0]); i <= i1; ++i)
+          for (int j = d > 1 ? pcell(1, a[1]) : 0, j1 = d > 1 ? pcell(1, b[1]) : 0; j <= j1; ++j)
+            for (int k = d > 2 ? pcell(2, a[2]) : 0, k1 = d > 2 ? pcell(2, b[2]) : 0; k <= k1; ++k)
+              for (int m = pstart[pindex(i, j, k)]; m < pstart[pindex(i, j, k) + 1]; ++m) {
+                const double* x = xyz + 3 * (size_t)pitem[m];
+                bool in = true;
+                for (int c = 0; c < d; ++c) in &= x[c] >= a[c] && x[c] <= b[c];
+                if (in) f.hits.push_back({pitem[m], e});
+              }
+      }
+    } catch (...) {
+      f.err = std::current_exception();
+    }
+  });
+  double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300};
+  std::vector<std::vector<int64_t>> cand(n);
+  for (auto& f : found) {  // ranges in element order, so every point's candidates ascend
+    if (f.err) std::rethrow_exception(f.err);
+    for (int c = 0; c < 3; ++c) {
+      lo[c] = std::min(lo[c], f.lo[c]);
+      hi[c] = std::max(hi[c], f.hi[c]);
+    }
+    for (auto& h : f.hits) cand[h.p].push_back(h.e);
+  }
   int g[3] = {1, 1, 1};
   const int gd = (int)std::max(1.0, std::floor(std::pow((double)K, 1.0 / d)));
   for (int c = 0; c < d; ++c) g[c] = gd;
@@ -466,54 +548,32 @@ std::vector<int64_t> locate_points(const RefElem& R, const double* node_xyz, int
     int i = span > 0 ? (int)std::floor((q - lo[c]) / span * g[c]) : 0;
     return std::min(std::max(i, 0), g[c] - 1);
   };
-  // bin elements (CSR over cells)
-  const int64_t ncell = (int64_t)g[0] * g[1] * g[2];
-  std::vector<int64_t> cnt(ncell + 1, 0);
-  std::vector<std::array<int, 6>> box(K);
-  for (int64_t e = 0; e < K; ++e) {
-    double a[3], b[3];
-    for (int c = 0; c < 3; ++c) {
-      a[c] = b[c] = node_xyz[((size_t)e * Np) * 3 + c];
-      for (int v = 1; v <= d; ++v) {
-        a[c] = std::min(a[c], node_xyz[((size_t)e * Np + v) * 3 + c]);
-        b[c] = std::max(b[c], node_xyz[((size_t)e * Np + v) * 3 + c]);
-      }
-    }
-    for (int c = 0; c < 3; ++c) {
-      const double tol = 1e-9 * (1 + hi[c] - lo[c]);
-      box[e][c] = cell(c, a[c] - tol);
-      box[e][3 + c] = cell(c, b[c] + tol);
-    }
-    for (int i = box[e][0]; i <= box[e][3]; ++i)
-      for (int j = box[e][1]; j <= box[e][4]; ++j)
-        for (int k = box[e][2]; k <= box[e][5]; ++k) ++cnt[((int64_t)i * g[1] + j) * g[2] + k + 1];
-  }
-  for (int64_t c = 0; c < ncell; ++c) cnt[c + 1] += cnt[c];
-  std::vector<int64_t> items(cnt[ncell]), fill(cnt.begin(), cnt.end() - 1);
-  for (int64_t e = 0; e < K; ++e)
-    for (int i = box[e][0]; i <= box[e][3]; ++i)
-      for (int j = box[e][1]; j <= box[e][4]; ++j)
-        for (int k = box[e][2]; k <= box[e][5]; ++k) items[fill[((int64_t)i * g[1] + j) * g[2] + k]++] = e;
-  for (int p = 0; p < n; ++p) {
-    const double* x = xyz + 3 * p;
+  auto locate = [&](int p) {
+    const double* x = xyz + 3 * (size_t)p;
     int64_t best = -1;
     double best_score = -1e300, best_l[4] = {0, 0, 0, 0}, l[4];
     bool in_box = true;
     for (int c = 0; c < d; ++c)
       if (x[c] < lo[c] - 1e-9 * (1 + hi[c] - lo[c]) || x[c] > hi[c] + 1e-9 * (1 + hi[c] - lo[c])) in_box = false;
-    if (in_box) {
-      const int64_t ci = ((int64_t)cell(0, x[0]) * g[1] + cell(1, x[1])) * g[2] + cell(2, x[2]);
-      for (int64_t it = cnt[ci]; it < cnt[ci + 1]; ++it) {
-        const double sc = bary_score(d, Np, node_xyz, items[it], x, l);
-        if (sc > best_score || (sc == best_score && items[it] < best)) {
-          best_score = sc;
-          best = items[it];
-          std::copy(l, l + 4, best_l);
-        }
+    for (size_t i = 0; in_box && i < cand[p].size(); ++i) {
+      const int64_t e = cand[p][i];
+      double a[3], b[3];
+      bounds(e, a, b);
+      bool meets = true;
+      for (int c = 0; c < d; ++c) {
+        const double tol = 1e-9 * (1 + hi[c] - lo[c]);
+        const int at = cell(c, x[c]);
+        meets &= cell(c, a[c] - tol) <= at && at <= cell(c, b[c] + tol);
+      }
+      if (!meets) continue;
+      const double sc = bary_score(d, Np, node_xyz, e, x, l);
+      if (sc > best_score) {
+        best_score = sc;
+        best = e;
+        std::copy(l, l + 4, best_l);
       }
     }
-    if (best < 0 || best_score < -1e-6)
-      throw InvalidArg("receiver point " + std::to_string(p) + " lies outside the mesh");
+    if (best < 0 || best_score < -1e-6) return;
     std::array<ld, 3> ref{0, 0, 0};
     if (d == 1) ref[0] = best_l[1] - best_l[0];
     else
@@ -522,24 +582,39 @@ std::vector<int64_t> locate_points(const RefElem& R, const double* node_xyz, int
     R.eval_basis(ref, phi.data(), nullptr);
     for (int k = 0; k < Np; ++k) w[(size_t)p * Np + k] = (double)phi[k];
     out[p] = best;
-  }
+  };
+  std::vector<std::exception_ptr> errs(8);
+  parallel_ranges(n, 8, [&](int t, int64_t p0, int64_t p1) {
+    try {
+      for (int64_t p = p0; p < p1; ++p) locate((int)p);
+    } catch (...) {
+      errs[t] = std::current_exception();
+    }
+  });
+  for (auto& e : errs)
+    if (e) std::rethrow_exception(e);
+  for (int p = 0; p < n; ++p)
+    if (out[p] < 0) throw InvalidArg("receiver point " + std::to_string(p) + " lies outside the mesh");
   return out;
 }
 
-// Install receivers (element, weights) on the context, with room for cap recorded steps.
+// Install receivers (element, weights) on the context, with room for cap recorded steps. Buffers of
+// the same sizes are kept, and with them the captured steps that hold their addresses.
 void install_receivers(Ctx& c, const std::vector<int64_t>& elem, const std::vector<double>& w, int cap) {
   DGK_HIP(hipStreamSynchronize(c.stream));
-  c.free_receivers();
-  c.drop_graphs();
   const int n = (int)elem.size();
-  if (!n) return;
-  if (cap < 1) throw InvalidArg("receiver capacity must be positive");
+  if (n && cap < 1) throw InvalidArg("receiver capacity must be positive");
   std::vector<int64_t> base(n);
   for (int i = 0; i < n; ++i) base[i] = elem[i] * c.Np;
-  DGK_HIP(hipMalloc(&c.rec.base, n * sizeof(int64_t)));
-  DGK_HIP(hipMalloc(&c.rec.w, (size_t)n * c.Np * c.tsize));
-  DGK_HIP(hipMalloc(&c.rec.out, (size_t)n * cap * c.tsize));
-  DGK_HIP(hipMalloc(&c.rec.counter, 2 * sizeof(int)));
+  if (!n || n != c.rec.n || cap != c.rec.cap) {
+    c.free_receivers();
+    c.drop_graphs();
+    if (!n) return;
+    DGK_HIP(hipMalloc(&c.rec.base, n * sizeof(int64_t)));
+    DGK_HIP(hipMalloc(&c.rec.w, (size_t)n * c.Np * c.tsize));
+    DGK_HIP(hipMalloc(&c.rec.out, (size_t)n * cap * c.tsize));
+    DGK_HIP(hipMalloc(&c.rec.counter, 2 * sizeof(int)));
+  }
   c.rec.n = n;
   c.rec.cap = cap;
   DGK_HIP(hipMemcpy(c.rec.base, base.data(), n * sizeof(int64_t), hipMemcpyHostToDevice));
@@ -549,7 +624,8 @@ void install_receivers(Ctx& c, const std::vector<int64_t>& elem, const std::vect
     std::vector<float> wf(w.begin(), w.end());
     DGK_HIP(hipMemcpy(c.rec.w, wf.data(), wf.size() * sizeof(float), hipMemcpyHostToDevice));
   }
-  DGK_HIP(hipMemset(c.rec.counter, 0, 2 * sizeof(int)));
+  const int zero[2] = {0, 0};
+  DGK_HIP(hipMemcpy(c.rec.counter, zero, sizeof(zero), hipMemcpyHostToDevice));
 }
 
 // Put rows x rec.n host values back into a freshly installed record and continue after them.
@@ -703,28 +779,54 @@ double* staging(Ctx& c) {
 
 namespace {
 
-// Host u[4][K*Np] (FP64) <-> a device state buffer in the state precision and layout. FP64 field
-// planes are copied directly; otherwise through the FP64 staging planes and a conversion kernel.
-void upload_planes(Ctx& c, const double* u, void* dst) {
-  const size_t row = (size_t)c.K * c.Np * sizeof(double);
-  if (c.precision == DGK_FP64 && c.es == 1) {
-    DGK_HIP(hipMemcpy2DAsync(dst, c.PS * sizeof(double), u, row, row, 4, hipMemcpyHostToDevice, c.stream));
-    return;
+// A state of at most this many bytes goes through a slab that the kernels read and write themselves:
+// no copy commands, whose fixed cost is most of a small hand-over (2D order 2, 2146 elements, 412 KB:
+// dgk_rhs 125 -> 57 us). Half a slab in, half out.
+constexpr size_t kDirectBytes = (size_t)1 << 20;
+static_assert(kDirectBytes <= Slabs::kSlabBytes / 2, "a state in and a state out of one slab");
+double* slab_in(Slab& s) { return (double*)s.p; }
+double* slab_out(Slab& s) { return (double*)(s.p + Slabs::kSlabBytes / 2); }
+bool direct(const Slab& s, int64_t n) { return s.p && 4 * (size_t)n * sizeof(double) <= kDirectBytes; }
+
+// Host u[4][n] (FP64) -> nodes [off, off+n) of a device state buffer in the state precision and layout.
+// Asynchronous: u (or the slab) is read until the stream is synchronised.
+void upload_planes(Ctx& c, const double* u, void* dst, int64_t off, int64_t n, Slab& slab) {
+  uint16_t* lo = dst == c.U && c.comp ? c.Ulo : nullptr;
+  if (c.precision == DGK_FP64 && c.es == 1) {  // planes in the state's own precision
+    DGK_HIP(hipMemcpy2DAsync((double*)dst + off, c.PS * sizeof(double), u, n * sizeof(double), n * sizeof(double), 4,
+                             hipMemcpyHostToDevice, c.stream));
+  } else if (direct(slab, n)) {
+    memcpy(slab_in(slab), u, 4 * n * sizeof(double));
+    state_from_f64(c, slab_in(slab), n, dst, lo, off, n);
+  } else {
+    double* s = staging(c) + off;
+    DGK_HIP(hipMemcpy2DAsync(s, c.PS * sizeof(double), u, n * sizeof(double), n * sizeof(double), 4,
+                             hipMemcpyHostToDevice, c.stream));
+    state_from_f64(c, s, c.PS, dst, lo, off, n);
   }
-  double* s = staging(c);
-  DGK_HIP(hipMemcpy2DAsync(s, c.PS * sizeof(double), u, row, row, 4, hipMemcpyHostToDevice, c.stream));
-  state_from_f64(c, s, dst, dst == c.U && c.comp ? c.Ulo : nullptr, 0, c.K * c.Np);
 }
 
-void download_planes(Ctx& c, const void* src, double* u) {
-  const size_t row = (size_t)c.K * c.Np * sizeof(double);
-  if (c.precision == DGK_FP64 && c.es == 1) {
-    DGK_HIP(hipMemcpy2DAsync(u, row, src, c.PS * sizeof(double), row, 4, hipMemcpyDeviceToHost, c.stream));
-    return;
+// And back; synchronous. Planes beyond the live fields are zero.
+void download_planes(Ctx& c, const void* src, double* u, int64_t off, int64_t n, Slab& slab) {
+  const uint16_t* lo = src == c.U && c.comp ? c.Ulo : nullptr;
+  const int live = c.es > 1 ? c.es : 4;
+  if (direct(slab, n) && c.es > 1) {
+    state_to_f64(c, src, lo, slab_out(slab), n, off, n);
+    DGK_HIP(hipStreamSynchronize(c.stream));
+    memcpy(u, slab_out(slab), live * n * sizeof(double));
+  } else {
+    const double* s = (const double*)src + off;
+    if (c.precision != DGK_FP64 || c.es != 1) {
+      double* d = staging(c) + off;
+      state_to_f64(c, src, lo, d, c.PS, off, n);
+      s = d;
+    }
+    std::vector<Piece> p;
+    for (int q = 0; q < live; ++q)
+      p.push_back({(const char*)(s + q * c.PS), (char*)(u + q * n), n * sizeof(double)});
+    DGK_HIP(download(p, c.stream));
   }
-  double* s = staging(c);
-  state_to_f64(c, src, src == c.U && c.comp ? c.Ulo : nullptr, s, 0, c.K * c.Np);
-  DGK_HIP(hipMemcpy2DAsync(u, row, s, c.PS * sizeof(double), row, 4, hipMemcpyDeviceToHost, c.stream));
+  std::fill(u + live * n, u + 4 * n, 0.0);
 }
 
 }  // namespace
@@ -780,7 +882,8 @@ dgk_status dgk_set_state(dgk_ctx* c, const double* u) {
         DGK_HIP(hipMemsetAsync((char*)p + nq * c->PS * c->tsize, 0, (4 - nq) * c->PS * c->tsize, c->stream));
       if (c->Ulo) DGK_HIP(hipMemsetAsync(c->Ulo + nq * c->PS, 0, (4 - nq) * c->PS * sizeof(uint16_t), c->stream));
     }
-    upload_planes(*c, u, c->U);
+    Slab slab(c->stream);
+    upload_planes(*c, u, c->U, 0, c->K * c->Np, slab);
     DGK_HIP(hipStreamSynchronize(c->stream));
   });
 }
@@ -788,8 +891,8 @@ dgk_status dgk_set_state(dgk_ctx* c, const double* u) {
 dgk_status dgk_get_state(dgk_ctx* c, double* u) {
   if (!c || !u) return fail(c, DGK_ERR_INVALID, "NULL argument");
   return guarded(c, [&] {
-    download_planes(*c, c->U, u);
-    DGK_HIP(hipStreamSynchronize(c->stream));
+    Slab slab(c->stream);
+    download_planes(*c, c->U, u, 0, c->K * c->Np, slab);
   });
 }
 
@@ -935,8 +1038,10 @@ dgk_status dgk_rhs(dgk_ctx* c, const double* u, double* out, double dt) {
     const int nq = live_planes(c->dim, u, c->K * c->Np);
     const int es = c->es;
     if (es > 1) c->es = nq;  // the operand's own live fields, for this call only
+    const int64_t n = c->K * c->Np;
+    Slab slab(c->stream);
     try {
-      upload_planes(*c, u, c->V1);
+      upload_planes(*c, u, c->V1, 0, n, slab);
       StageArgs a = base_args(*c);
       a.dt = dt;
       a.stage = 4;
@@ -944,15 +1049,14 @@ dgk_status dgk_rhs(dgk_ctx* c, const double* u, double* out, double dt) {
       a.Vout = c->V0;
       a.nq = nq;
       launch_stage(*c, a, c->stream);
-      download_planes(*c, c->V0, out);
-      DGK_HIP(hipStreamSynchronize(c->stream));
+      download_planes(*c, c->V0, out, 0, n, slab);
     } catch (...) {
       c->es = es;
       throw;
     }
     c->es = es;
-    const int64_t n = c->K * c->Np;  // planes that are not live have a zero right-hand side
-    std::fill(out + nq * n, out + 4 * n, 0.0);
+    // planes that are not live have a zero right-hand side
+    if (es == 1) std::fill(out + nq * n, out + 4 * n, 0.0);
   });
 }
 
@@ -1254,7 +1358,6 @@ dgk_status batch_state_io(dgk_batch* b, int sim, double* u, bool to_device) {
     dgk::Ctx& c = *b->groups[w.first].ctx;
     DGK_HIP(hipStreamSynchronize(b->main));
     const int64_t off = b->groups[w.first].off[w.second] * c.Np, n = b->K[sim] * c.Np;
-    const bool f64 = c.precision == DGK_FP64;
     if (to_device) {  // the group's live planes: the most any member needs
       b->nq[sim] = dgk::live_planes(c.dim, u, n);
       int nq = c.dim + 1;
@@ -1266,27 +1369,15 @@ dgk_status batch_state_io(dgk_batch* b, int sim, double* u, bool to_device) {
         // interleaved buffers hold exactly the live fields: relay the whole group's state
         double* s = dgk::staging(c);
         uint16_t* lo = c.comp ? c.Ulo : nullptr;
-        dgk::state_to_f64(c, c.U, lo, s, 0, c.K * c.Np);
+        dgk::state_to_f64(c, c.U, lo, s, c.PS, 0, c.K * c.Np);
         c.es = nq;
-        dgk::state_from_f64(c, s, c.U, lo, 0, c.K * c.Np);
+        dgk::state_from_f64(c, s, c.PS, c.U, lo, 0, c.K * c.Np);
       }
       c.nq = nq;
     }
-    // FP64 field planes are copied directly; otherwise through the FP64 staging planes
-    const bool direct = f64 && c.es == 1;
-    double* s = direct ? nullptr : dgk::staging(c);
-    uint16_t* lo = c.comp ? c.Ulo : nullptr;
-    if (!to_device && !direct) dgk::state_to_f64(c, c.U, lo, s, off, n);
-    for (int q = 0; q < 4; ++q) {
-      const int64_t o = q * c.PS + off;
-      void* dev = direct ? (void*)((char*)c.U + o * c.tsize) : (void*)(s + o);
-      double* host = u + q * n;
-      if (to_device)
-        DGK_HIP(hipMemcpyAsync(dev, host, n * sizeof(double), hipMemcpyHostToDevice, c.stream));
-      else
-        DGK_HIP(hipMemcpyAsync(host, dev, n * sizeof(double), hipMemcpyDeviceToHost, c.stream));
-    }
-    if (to_device && !direct) dgk::state_from_f64(c, s, c.U, lo, off, n);
+    dgk::Slab slab(c.stream);
+    if (to_device) dgk::upload_planes(c, u, c.U, off, n, slab);
+    else dgk::download_planes(c, c.U, u, off, n, slab);
     DGK_HIP(hipStreamSynchronize(c.stream));
   });
 }

@@ -9,6 +9,7 @@
 #include <vector>
 
 #include "../../include/dgk.h"
+#include "handover.hpp"
 
 namespace dgk {
 
@@ -156,6 +157,7 @@ struct Ctx {
   int* tstep = nullptr;
   std::string err;
   std::vector<void*> allocs;
+  SlabUser slabs;
 
   void* alloc(size_t bytes) {
     void* p = nullptr;
@@ -182,11 +184,11 @@ void launch_source(Ctx& c, const Ctx::Src& s, double value, hipStream_t st);
 // hard source overwrite at the step whose start time is c.tdev[*c.tstep] (when t < duration) and ++*c.tstep
 void launch_edge(Ctx& c, bool record, bool source, hipStream_t st);
 bool check_finite(Ctx& c);
-// FP64 field planes on the device (plane stride PS; element nodes [off, off+n) of each plane) -> a
+// FP64 field planes s[q*stride + i], i < n (device or page-locked host memory) -> nodes [off, off+n) of a
 // state buffer in the context's precision and layout; in the FP32 compensated form lo (if given)
 // receives the bf16 low words. And back, adding the low words when lo is given.
-void state_from_f64(Ctx& c, const double* s_dev, void* dst_dev, uint16_t* lo, int64_t off, int64_t n);
-void state_to_f64(Ctx& c, const void* src_dev, const uint16_t* lo, double* s_dev, int64_t off, int64_t n);
+void state_from_f64(Ctx& c, const double* s, int64_t stride, void* dst_dev, uint16_t* lo, int64_t off, int64_t n);
+void state_to_f64(Ctx& c, const void* src_dev, const uint16_t* lo, double* s, int64_t stride, int64_t off, int64_t n);
 const char* variant_name(int v);
 // MFMA k-steps, 16-row blocks and 4-row tail pieces (0: none) of the stage kernel's operator
 void mfma_shape(int dim, int p, bool fp32, bool oplo, int* KS, int* MB, int* NT);

@@ -1033,30 +1033,30 @@ __global__ void k_finite(const T* __restrict__ x, int64_t n, int* __restrict__ f
   if (__any(bad) && (threadIdx.x % 64) == 0) atomicOr(flag, 1);
 }
 
-// FP64 field planes (plane stride PS; element nodes [off, off+n) of each plane) -> a state buffer in
-// the context's precision and layout (es > 1: node-interleaved with es fields, the planes beyond es
-// being zero; es = 1: planes), with the bf16 low word of the FP32 remainder when lo is given; and
-// back (planes beyond es come back as zero).
+// FP64 field planes s[q*SS + i] of the n nodes [off, off+n) -> a state buffer in the context's precision
+// and layout (es > 1: node-interleaved with es fields, the planes beyond es being zero; es = 1: planes of
+// stride PS), with the bf16 low word of the FP32 remainder when lo is given; and back (planes beyond es
+// come back as zero). s may be page-locked host memory.
 __device__ __forceinline__ void field_node(int64_t i, int64_t n, int64_t off, int es, int64_t PS, int64_t* q,
-                                           int64_t* node, int64_t* di) {
+                                           int64_t* local, int64_t* di) {
   if (es > 1) {
     *q = i & 3;
-    *node = off + (i >> 2);
-    *di = *node * es + *q;
+    *local = i >> 2;
+    *di = (off + *local) * es + *q;
   } else {
     *q = i / n;
-    *node = off + (i - *q * n);
-    *di = *q * PS + *node;
+    *local = i - *q * n;
+    *di = *q * PS + off + *local;
   }
 }
 template <typename T>
-__global__ void k_from_f64(const double* __restrict__ s, int64_t PS, int64_t off, int64_t n, T* __restrict__ d,
-                           uint16_t* __restrict__ lo, int es) {
+__global__ void k_from_f64(const double* __restrict__ s, int64_t SS, int64_t PS, int64_t off, int64_t n,
+                           T* __restrict__ d, uint16_t* __restrict__ lo, int es) {
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < 4 * n; i += (int64_t)gridDim.x * blockDim.x) {
-    int64_t q, node, di;
-    field_node(i, n, off, es, PS, &q, &node, &di);
+    int64_t q, local, di;
+    field_node(i, n, off, es, PS, &q, &local, &di);
     if (es > 1 && q >= es) continue;
-    const double x = s[q * PS + node];
+    const double x = s[q * SS + local];
     if constexpr (sizeof(T) == 8) {
       d[di] = x;
     } else {
@@ -1067,12 +1067,12 @@ __global__ void k_from_f64(const double* __restrict__ s, int64_t PS, int64_t off
   }
 }
 template <typename T>
-__global__ void k_to_f64(const T* __restrict__ d, const uint16_t* __restrict__ lo, int64_t PS, int64_t off, int64_t n,
-                         double* __restrict__ s, int es) {
+__global__ void k_to_f64(const T* __restrict__ d, const uint16_t* __restrict__ lo, int64_t SS, int64_t PS, int64_t off,
+                         int64_t n, double* __restrict__ s, int es) {
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < 4 * n; i += (int64_t)gridDim.x * blockDim.x) {
-    int64_t q, node, di;
-    field_node(i, n, off, es, PS, &q, &node, &di);
-    s[q * PS + node] = (es > 1 && q >= es) ? 0.0 : (double)d[di] + (lo ? (double)bf16_bits_to_f32(lo[di]) : 0.0);
+    int64_t q, local, di;
+    field_node(i, n, off, es, PS, &q, &local, &di);
+    s[q * SS + local] = (es > 1 && q >= es) ? 0.0 : (double)d[di] + (lo ? (double)bf16_bits_to_f32(lo[di]) : 0.0);
   }
 }
 
@@ -1329,24 +1329,25 @@ bool check_finite(Ctx& c) {
   return h == 0;
 }
 
-void state_from_f64(Ctx& c, const double* s, void* dst, uint16_t* lo, int64_t off, int64_t n) {
-  const int es = c.es;
+void state_from_f64(Ctx& c, const double* s, int64_t stride, void* dst, uint16_t* lo, int64_t off, int64_t n) {
+  const unsigned nb = (unsigned)std::max<int64_t>(1, std::min<int64_t>(1024, (4 * n + 255) / 256));
   if (c.precision == DGK_FP64)
-    hipLaunchKernelGGL(k_from_f64<double>, dim3(1024), dim3(256), 0, c.stream, s, c.PS, off, n, (double*)dst,
-                       (uint16_t*)nullptr, es);
+    hipLaunchKernelGGL(k_from_f64<double>, dim3(nb), dim3(256), 0, c.stream, s, stride, c.PS, off, n, (double*)dst,
+                       (uint16_t*)nullptr, c.es);
   else
-    hipLaunchKernelGGL(k_from_f64<float>, dim3(1024), dim3(256), 0, c.stream, s, c.PS, off, n, (float*)dst, lo, es);
+    hipLaunchKernelGGL(k_from_f64<float>, dim3(nb), dim3(256), 0, c.stream, s, stride, c.PS, off, n, (float*)dst, lo,
+                       c.es);
   DGK_HIP(hipGetLastError());
 }
 
-void state_to_f64(Ctx& c, const void* src, const uint16_t* lo, double* s, int64_t off, int64_t n) {
-  const int es = c.es;
+void state_to_f64(Ctx& c, const void* src, const uint16_t* lo, double* s, int64_t stride, int64_t off, int64_t n) {
+  const unsigned nb = (unsigned)std::max<int64_t>(1, std::min<int64_t>(1024, (4 * n + 255) / 256));
   if (c.precision == DGK_FP64)
-    hipLaunchKernelGGL(k_to_f64<double>, dim3(1024), dim3(256), 0, c.stream, (const double*)src,
-                       (const uint16_t*)nullptr, c.PS, off, n, s, es);
+    hipLaunchKernelGGL(k_to_f64<double>, dim3(nb), dim3(256), 0, c.stream, (const double*)src,
+                       (const uint16_t*)nullptr, stride, c.PS, off, n, s, c.es);
   else
-    hipLaunchKernelGGL(k_to_f64<float>, dim3(1024), dim3(256), 0, c.stream, (const float*)src, lo, c.PS, off, n, s,
-                       es);
+    hipLaunchKernelGGL(k_to_f64<float>, dim3(nb), dim3(256), 0, c.stream, (const float*)src, lo, stride, c.PS, off, n,
+                       s, c.es);
   DGK_HIP(hipGetLastError());
 }
 

@@ -21,6 +21,7 @@
 #include <vector>
 
 #include "../../include/dgk_surrogate.h"
+#include "handover.hpp"
 
 // Scratch of the allocation-free forward pass (dgs_forward_noalloc): one copy per GPU, held until
 // the process ends. Host code never uses this name as an address; it uses the per-device pointer
@@ -447,6 +448,7 @@ struct Net {
   int64_t ndata = 0;
   std::vector<void*> allocs;
   std::string err;
+  dgk::SlabUser slabs;
 
   template <typename U>
   U* alloc(size_t n) {
@@ -791,17 +793,38 @@ dgs_status dgs_forward(dgs_net* n, int rows, const float* x, float* y) {
   if (!n || rows < 0 || (rows && (!x || !y))) return DGS_ERR_INVALID;
   return dgs::guarded(n, [&] {
     const int mb = n->cfg.max_batch, in = n->cfg.in_dim, No = n->cfg.out_dim;
-    std::vector<float> xb((size_t)mb * in);
+    // few rows: the kernels read the inputs and write the outputs in a page-locked slab themselves (half
+    // of it each), without copy commands (100 rows, 2048 outputs: 124 -> 78 us); otherwise the slab only
+    // carries the inputs
+    constexpr size_t half = dgk::Slabs::kSlabBytes / 2, most = (size_t)2 << 20;
+    dgk::Slab slab(n->s);
     for (int r0 = 0; r0 < rows; r0 += mb) {
       const int m = std::min(mb, rows - r0);
-      const int mp = (m + 63) / 64 * 64;  // pad to whole 64-row tiles with copies of the last row
-      for (int r = 0; r < mp; ++r)
-        std::copy(x + (size_t)(r0 + std::min(r, m - 1)) * in, x + (size_t)(r0 + std::min(r, m - 1) + 1) * in,
-                  xb.begin() + (size_t)r * in);
-      dgs::upload_rows(*n, mp, xb.data(), nullptr, nullptr);
-      dgs::forward(*n, mp);
-      DGS_HIP(hipMemcpyAsync(y + (size_t)r0 * No, n->y, (size_t)m * No * sizeof(float), hipMemcpyDeviceToHost, n->s));
-      DGS_HIP(hipStreamSynchronize(n->s));
+      const int mp = (m + 63) / 64 * 64;  // whole 64-row tiles, padded with copies of the last row
+      const size_t xbytes = (size_t)m * in * sizeof(float), ybytes = (size_t)m * No * sizeof(float);
+      dgs::Pass b{};
+      b.m = m;
+      b.z = n->z;
+      b.hl = &n->h;
+      b.prel = &n->pre;
+      b.y = n->y;
+      if (slab.p && xbytes <= half) {
+        memcpy(slab.p, x + (size_t)r0 * in, xbytes);
+        b.x = (const float*)slab.p;
+      } else {
+        DGS_HIP(hipMemcpyAsync(n->x, x + (size_t)r0 * in, xbytes, hipMemcpyHostToDevice, n->s));
+        b.x = n->x;
+      }
+      const bool direct = slab.p && ybytes <= most;
+      if (direct) b.y = (float*)(slab.p + half);
+      dgs::forward(*n, mp, b);
+      float* to = y + (size_t)r0 * No;
+      if (direct) {
+        DGS_HIP(hipStreamSynchronize(n->s));
+        memcpy(to, b.y, ybytes);
+      } else {
+        DGS_HIP(dgk::download({{(const char*)n->y, (char*)to, ybytes}}, n->s));
+      }
     }
   });
 }

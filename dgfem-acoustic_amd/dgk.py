@@ -317,7 +317,7 @@ class Solver:
         self._check(device().dgk_set_state(self.h, _p(u)))
 
     def get_state(self):
-        u = np.zeros((4, self.K * self.Np))
+        u = np.empty((4, self.K * self.Np))
         self._check(device().dgk_get_state(self.h, _p(u)))
         return u
 
@@ -335,7 +335,7 @@ class Solver:
 
     def rhs(self, u, dt):
         u = np.ascontiguousarray(u, dtype=np.float64)
-        out = np.zeros_like(u)
+        out = np.empty_like(u)
         self._check(device().dgk_rhs(self.h, _p(u), _p(out), float(dt)))
         return out
 
@@ -437,7 +437,7 @@ class Batch:
 
     def get_state(self, i):
         m = self.meshes[i]
-        u = np.zeros((4, m.K * m.Np))
+        u = np.empty((4, m.K * m.Np))
         self._check(device().dgk_batch_get_state(self.h, int(i), _p(u)))
         return u
 

@@ -104,7 +104,7 @@ class Net:
 
     def forward(self, x):
         xa, xp = _f(x)
-        y = np.zeros((len(xa), self.cfg["out_dim"]), np.float32)
+        y = np.empty((len(xa), self.cfg["out_dim"]), np.float32)
         self._check(_lib().dgs_forward(self.h, len(xa), xp, y.ctypes.data_as(_P(ctypes.c_float))), "dgs_forward")
         return y
 
