@@ -669,35 +669,37 @@ __global__ __launch_bounds__((MfmaLaunch<T, D, P, SH>::KB), (MfmaLaunch<T, D, P,
 #pragma unroll
     for (int t = 0; t < NFC; ++t)
       if (gtid + t * GT < GE * NF * 4) sN[grp * GE * NF * 4 + gtid + t * GT] = pfg[t];
-    // epilogue operands: issued here, a tile ahead of their use, when registers allow; shapes with
-    // the operator in global memory load them just before the epilogue instead
-    VT pu[NE], pa[NE];
+    // Epilogue operands. pe: u_n (at stage 3 without the compensated solution: W); pa: the accumulator.
+    // They are touched once per stage per element, and on large meshes more than the caches hold passes
+    // before their next use: their loads and stores carry the non-temporal hint, which leaves the caches
+    // to the neighbour traces and stage inputs (1-3% per stage on the HBM-bound shapes).
+    // Without the compensated solution the stage inputs V1 = u + k1/2, V2 = u + k2/2 and V3 = u + k3 hold
+    // the increments, u_new = (V1 + 2 V2 + V3 - u)/3 + k4/6: stage 1, which has u, V1 (its input) and V2
+    // (its output), stores W = V1 + 2 V2 - u, and stage 3 adds V3 (its input) and k4. 12 state words per
+    // unknown and step are moved instead of 16 with a running accumulator, no stage loads more than one
+    // array beside its input, and u is rounded fewer times (V1, V2, V3 enter with weights 1/3, 2/3 and
+    // 1/3, W with 2/3; differences come first and are exact where the increments are small).
+    // us per stage in graph replay, 13 words (with A = u + (k1 + 2 k2 + 2 k3)/6 formed at stage 2 from V1)
+    // -> 12: 2D order 2 FP64, 179,998 elements, 29.5 -> 28.9; 3D order 4, 48,000, 62.6 -> 60.2; order 5,
+    // 7722, 31.6 -> 31.0 (16 -> 13: 36.9 -> 35.4 at 2D order 2).
+    VT pe[NE], pa[CS ? NE : 1];
     uint2 plo[CS ? NE : 1];
-    // u_n and the accumulator are touched once per stage per element, and on large meshes more
-    // than the caches hold passes before their next use: their loads and stores carry the
-    // non-temporal hint, which leaves the caches to the neighbour traces and stage inputs (1-3% per
-    // stage on the HBM-bound shapes)
-    // Without the compensated solution the accumulator of stages 0 and 1 is not stored: the stage
-    // inputs V1 = u + k1/2 and V2 = u + k2/2 already hold k1 and k2, so stage 2 (whose input is V2
-    // and whose output V3 replaces V1) forms A = u + ((V1 - u) + 2 (V2 - u) + k3) / 3 and stage 3
-    // adds k4/6. 13 state words per unknown and step are moved instead of 16, and u is rounded
-    // fewer times (A once instead of three times; V1 and V2 enter with weights 1/3 and 2/3).
-    // 2D order 2 FP64, 179,998 elements: 36.9 -> 35.4 us per stage; 3D order 3 FP64, 196,608: 131 -> 129.
     auto load_epi = [&]() {
-    if (stage >= 1 && stage <= 3) {
+      if (stage < 1 || stage > 3) return;
+      const T* const p = !CS && stage == 3 ? (const T*)Acc : (const T*)U;
 #pragma unroll
       for (int t = 0; t < NE; ++t)
         if (has_vec(t)) {
-          if (stage != 3 || CS) pu[t] = __builtin_nontemporal_load((const VT*)tile_at(U, e0, NP * ES, voff[t]));
-          if (CS && stage == 3) plo[CS ? t : 0] = *(const uint2*)tile_at(Ulo, e0, NP * ES, voff[t]);
-          if (CS || stage != 1)
-            pa[t] = __builtin_nontemporal_load(
-                (const VT*)tile_at(!CS && stage == 2 ? (const T*)Vout : (const T*)Acc, e0, NP * ES, voff[t]));
+          pe[t] = __builtin_nontemporal_load((const VT*)tile_at(p, e0, NP * ES, voff[t]));
+          if constexpr (CS) {
+            pa[t] = __builtin_nontemporal_load((const VT*)tile_at((const T*)Acc, e0, NP * ES, voff[t]));
+            if (stage == 3) plo[t] = *(const uint2*)tile_at(Ulo, e0, NP * ES, voff[t]);
+          }
         }
-    }
     };
-    // wide workgroups and operators read from global memory need the registers during the MFMA
-    // chain: their epilogue operands are loaded later (below)
+    // Issued here, a tile ahead of their use, when registers allow. Wide workgroups and shapes 9-11 need
+    // the registers during the MFMA chain and load them after its volume k-steps; with the operator in
+    // global memory they come just before the epilogue.
     constexpr bool kDefer = !kALds || MfmaLaunch<T, D, P, SH>::WAVES > 4 || MfmaLaunch<T, D, P, SH>::DEFER;
     if (!kDefer) load_epi();
     cnc = inc;
@@ -784,14 +786,11 @@ __global__ __launch_bounds__((MfmaLaunch<T, D, P, SH>::KB), (MfmaLaunch<T, D, P,
     // block of the row split)
     auto chain = [&](auto astride) {
       constexpr int AS = decltype(astride)::value;
-      auto step = [&](const int s, const T b) {
-#pragma unroll
-        for (int mb = 0; mb < MBW; ++mb) {
-          const int ai = NCH > 1 ? mb * NCH + (s & 1) : mb;
-          acc[ai] = Mfma<T>::mma(pAt[(mb * KS + s) * AS], b, acc[ai]);
-        }
-#pragma unroll
-        for (int t = 0; t < NT4; ++t) acct[t] = Tail<T>::mma(pTt[(t * KS + s) * 16], b, acct[t]);
+      auto mma = [&](const int s, const int mb, const T a, const T b) {
+        const int ai = NCH > 1 ? mb * NCH + (s & 1) : mb;
+        acc[ai] = Mfma<T>::mma(a, b, acc[ai]);
+      };
+      auto low = [&](const int s, const T b) {
         if constexpr (LO) {
           blo[s % 8] = (__bf16)b;
           if (s % 8 == 7 || s == KS - 1) {
@@ -803,30 +802,87 @@ __global__ __launch_bounds__((MfmaLaunch<T, D, P, SH>::KB), (MfmaLaunch<T, D, P,
           }
         }
       };
-      constexpr int kNodeUnroll = kALds ? NG : 2;
-#pragma unroll kNodeUnroll
-      for (int m = 0; m < NG; ++m) {
+      constexpr int NV = D * NG;  // volume k-steps
+      // fields of node 4m + g of the lane's element (zero beyond the last node)
+      auto load_nodes = [&](const int m, T f[4]) {
         const int n = 4 * m + g;
-        T p = 0, vx = 0, vy = 0, vz = 0;
-        if (n < NP) {
-          T f[4];
-          node_fields<ES>(sU + el * LES + n * ES, f);
-          p = f[0];
-          vx = f[1];
-          vy = f[2];
-          vz = f[3];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) f[c] = 0;
+        if (n < NP) node_fields<ES>(sU + el * LES + n * ES, f);
+      };
+      auto load_face = [&](const int s) {
+        const int jk = 4 * (s - NV) + g;
+        return jk < NFF ? sB[(el * 4 + q) * RB + jk] : (T)0;
+      };
+      auto volume = [&](const int r, const T f[4]) {
+        T v = alpha[r] * f[0];  // explicitly fused, so that every form of the chain rounds alike
+#pragma unroll
+        for (int c = 1; c < ES; ++c) v = fma(beta[r][c - 1], f[c], v);
+        return v;
+      };
+      if constexpr (kALds && !(sizeof(T) == 8 && D == 3)) {
+        // Software pipeline, one region of the schedule per k-step: the first MFMA of k-step s is
+        // issued, then (in its shadow) the LDS reads of the operator and face values PF k-steps
+        // ahead and of the next node group, and the B value of k-step s+1, then the other MFMAs of
+        // k-step s. The fences keep the compiler from sinking the reads back to their uses, where
+        // every k-step waits for the LDS latency. FP64 holds one k-step ahead (its registers), and in
+        // 3D none: order 3 would spill 49 registers (105 -> 261 us per stage, 196,608 elements), order 5
+        // loses 2%. us per stage in graph replay, unrolled loop -> pipeline: 2D order 3 FP64, 500,000
+        // elements, 100.7 -> 96.5; order 4, 320,000, 88.5 -> 82.4; FP32 2D order 2, 980,000, 97.2 -> 95.0;
+        // 3D order 5, 82,944, 118 -> 113; order 3, 196,608, 66.5 -> 65.5.
+        constexpr int PF = sizeof(T) == 4 ? 4 : 1, NS = PF + 1;
+        T fn[2][4], af[NS][MBW ? MBW : 1], tf[NS][NT4 ? NT4 : 1], ff[NS];
+        auto load_op = [&](const int s) {
+#pragma unroll
+          for (int mb = 0; mb < MBW; ++mb) af[s % NS][mb] = pAt[(mb * KS + s) * AS];
+#pragma unroll
+          for (int t = 0; t < NT4; ++t) tf[s % NS][t] = pTt[(t * KS + s) * 16];
+          if (s >= NV) ff[s % NS] = load_face(s);
+        };
+        load_nodes(0, fn[0]);
+#pragma unroll
+        for (int s = 0; s < PF && s < KS; ++s) load_op(s);
+        T b = volume(0, fn[0]);
+#pragma unroll
+        for (int s = 0; s < KS; ++s) {
+          if constexpr (MBW > 0) mma(s, 0, af[s % NS][0], b);
+          __builtin_amdgcn_sched_barrier(0);
+          if (s + PF < KS) load_op(s + PF);
+          if (s < NV && s % D == 0 && s / D + 1 < NG) load_nodes(s / D + 1, fn[(s / D + 1) & 1]);
+          T bn = 0;
+          if (s + 1 < NV) bn = volume((s + 1) % D, fn[((s + 1) / D) & 1]);
+          else if (s + 1 < KS) bn = ff[(s + 1) % NS];
+          if (kDefer && s == NV - 1) load_epi();
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int mb = 1; mb < MBW; ++mb) mma(s, mb, af[s % NS][mb], b);
+#pragma unroll
+          for (int t = 0; t < NT4; ++t) acct[t] = Tail<T>::mma(tf[s % NS][t], b, acct[t]);
+          low(s, b);
+          __builtin_amdgcn_sched_barrier(0);
+          b = bn;
         }
+      } else {
+        auto step = [&](const int s, const T b) {
 #pragma unroll
-        for (int r = 0; r < D; ++r)
-          step(m * D + r, alpha[r] * p + beta[r][0] * vx + beta[r][1] * vy + beta[r][2] * vz);
-      }
-      // 8-wave workgroups: the epilogue operands are issued here, in flight during the face k-steps
-      // (the volume coefficients are dead by now, which keeps the peak within 256 registers)
-      if (kDefer && kALds) load_epi();
+          for (int mb = 0; mb < MBW; ++mb) mma(s, mb, pAt[(mb * KS + s) * AS], b);
 #pragma unroll
-      for (int f = 0; f < NFK; ++f) {
-        const int jk = 4 * f + g;
-        step(D * NG + f, jk < NFF ? sB[(el * 4 + q) * RB + jk] : (T)0);
+          for (int t = 0; t < NT4; ++t) acct[t] = Tail<T>::mma(pTt[(t * KS + s) * 16], b, acct[t]);
+          low(s, b);
+        };
+        constexpr int kNodeUnroll = kALds ? NG : 2;
+#pragma unroll kNodeUnroll
+        for (int m = 0; m < NG; ++m) {
+          T f[4];
+          load_nodes(m, f);
+#pragma unroll
+          for (int r = 0; r < D; ++r) step(m * D + r, volume(r, f));
+        }
+        // in flight during the face k-steps (the volume coefficients are dead by now, which keeps the
+        // peak within 256 registers)
+        if (kDefer && kALds) load_epi();
+#pragma unroll
+        for (int f = 0; f < NFK; ++f) step(NV + f, load_face(NV + f));
       }
     };
     if constexpr (kCompact) {
@@ -881,18 +937,19 @@ __global__ __launch_bounds__((MfmaLaunch<T, D, P, SH>::KB), (MfmaLaunch<T, D, P,
           if constexpr (CS) __builtin_nontemporal_store(kq * s6, pAcc);
           *pOut = u + kq * s2;
         } break;
-        case 1:
-          if constexpr (CS) __builtin_nontemporal_store(pa[t] + kq * s3, pAcc);
-          *pOut = pu[t] + kq * s2;
-          break;
-        case 2:
+        case 1: {
+          const VT u = pe[t], v2 = u + kq * s2;
           if constexpr (CS) {
             __builtin_nontemporal_store(pa[t] + kq * s3, pAcc);
           } else {
-            const VT u = pu[t], v2 = *(const VT*)(sU + loff[t]);
-            __builtin_nontemporal_store(u + ((pa[t] - u) + (v2 - u) * (T)2 + kq) * s3, pAcc);
+            const VT v1 = *(const VT*)(sU + loff[t]);
+            __builtin_nontemporal_store(u * (T)2 + ((v1 - u) + (v2 - u) * (T)2), pAcc);
           }
-          *pOut = pu[t] + kq;
+          *pOut = v2;
+        } break;
+        case 2:
+          if constexpr (CS) __builtin_nontemporal_store(pa[t] + kq * s3, pAcc);
+          *pOut = pe[t] + kq;
           break;
         case 3:
           if constexpr (CS) {
@@ -903,7 +960,7 @@ __global__ __launch_bounds__((MfmaLaunch<T, D, P, SH>::KB), (MfmaLaunch<T, D, P,
             uint32_t ob[4];
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-              const float u = pu[t][i], x = d[i];
+              const float u = pe[t][i], x = d[i];
               const float sum = u + x, bv = sum - u;
               const float err = (u - (sum - bv)) + (x - bv);  // two-sum: u + x = sum + err exactly
               const float lo = bf16_bits_to_f32(lb[i]) + err;
@@ -914,7 +971,8 @@ __global__ __launch_bounds__((MfmaLaunch<T, D, P, SH>::KB), (MfmaLaunch<T, D, P,
             __builtin_nontemporal_store(hi, pU);
             *pLo = make_uint2(ob[0] | (ob[1] << 16), ob[2] | (ob[3] << 16));
           } else {
-            __builtin_nontemporal_store(pa[t] + kq * s6, pU);
+            const VT v3 = *(const VT*)(sU + loff[t]);
+            __builtin_nontemporal_store(v3 + ((pe[t] - v3 * (T)2) * s3 + kq * s6), pU);
           }
           break;
         case 4: *pOut = kq; break;
