@@ -300,8 +300,8 @@ void create_impl(Ctx& c, const dgk_mesh* m, const dgk_phys* ph, const dgk_opts* 
   c.A = c.alloc(n * c.tsize);
   c.V0 = c.alloc(n * c.tsize);
   c.V1 = c.alloc(n * c.tsize);
-  c.Jinv = c.alloc(KP * 9 * c.tsize);
-  c.fgeom = c.alloc(KP * c.Nf * 4 * c.tsize);
+  c.Jinv = c.alloc(KP * c.dim * c.dim * c.tsize);
+  c.fgeom = c.alloc(KP * c.Nf * (c.dim + 1) * c.tsize);
   c.nbr = (int32_t*)c.alloc(KP * c.Nf * sizeof(int32_t));
   c.code = (int32_t*)c.alloc(KP * c.Nf * sizeof(int32_t));
   c.nface = (int32_t*)c.alloc(KP * c.Nf * sizeof(int32_t));
@@ -313,8 +313,8 @@ void create_impl(Ctx& c, const dgk_mesh* m, const dgk_phys* ph, const dgk_opts* 
     c.Ulo = (uint16_t*)c.alloc(n * sizeof(uint16_t));
     DGK_HIP(hipMemsetAsync(c.Ulo, 0, n * sizeof(uint16_t), c.stream));
   }
-  DGK_HIP(hipMemsetAsync(c.Jinv, 0, KP * 9 * c.tsize, c.stream));
-  DGK_HIP(hipMemsetAsync(c.fgeom, 0, KP * c.Nf * 4 * c.tsize, c.stream));
+  DGK_HIP(hipMemsetAsync(c.Jinv, 0, KP * c.dim * c.dim * c.tsize, c.stream));
+  DGK_HIP(hipMemsetAsync(c.fgeom, 0, KP * c.Nf * (c.dim + 1) * c.tsize, c.stream));
   DGK_HIP(hipMemsetAsync(c.nbr, 0xff, KP * c.Nf * sizeof(int32_t), c.stream));
   DGK_HIP(hipMemsetAsync(c.code, 0, KP * c.Nf * sizeof(int32_t), c.stream));
   double* vx = nullptr;

@@ -39,7 +39,7 @@ constexpr int kTilePad = 32;  // device arrays hold a multiple of this many elem
 constexpr int kVariantLds = 1;   // thread per element node, operators read from memory
 constexpr int kVariantMfma = 2;  // 16x16x4 MFMA contraction, one wave per 4 elements
 // The MFMA stage kernel addresses its arrays with 32-bit byte offsets from the buffers' own bases
-// while every one of them (state: Kpad*np*es values, J^-1: Kpad*9, face geometry: Kpad*nf*4) stays
+// while every one of them (state: Kpad*np*es values, J^-1: at most Kpad*9, face geometry: Kpad*nf*4) stays
 // below 4 GiB, and through 64-bit per-tile bases otherwise.
 inline bool stage_needs_addr64(int64_t Kpad, int np, int nf, int es, int tsize) {
   const uint64_t lim = (uint64_t)1 << 32, kp = (uint64_t)Kpad;
@@ -74,8 +74,8 @@ struct StageArgs {
   void* U;
   void* A;
   void* Ulo;              // FP32 compensated form: bf16 low word of U (uint16 bits), else null
-  const void* Jinv;       // [K][9]
-  const void* fgeom;      // [K][Nf][4]: unit outward normal, sJ/|detJ|
+  const void* Jinv;       // [K][dim][dim]
+  const void* fgeom;      // [K][Nf][dim + 1]: unit outward normal, sJ/|detJ|
   const int32_t* nbr;     // [K*Nf]
   const int32_t* code;    // [K*Nf]: (nbr_face*nperm + perm) | (penalty sign -1 ? 1<<16 : 0)
   const void* W;

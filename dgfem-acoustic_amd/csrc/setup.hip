@@ -137,15 +137,14 @@ __global__ void k_face_finalize(int64_t K, int D, int NF, int NPERM, const int32
   code[t] = (jn * NPERM + pidx) | (sign < 0 ? (1 << 16) : 0);
 }
 
-// Affine geometry: Jinv[r][x] = d r / d x (Gmsh reference coordinates), stored 3x3 row-major.
 struct FaceRef {
   double n[4][3];  // outward reference normals
   double fsc[4];   // reference face measure / face reference-element measure
 };
 
-// Affine geometry: Jinv[r][x] = d r / d x (Gmsh reference coordinates), stored 3x3 row-major,
-// and per element face the unit outward normal J^-T n_ref / |J^-T n_ref| and the face scale
-// sJ/|detJ| = |J^-T n_ref| * fsc, computed in FP64 and rounded once to T.
+// Affine geometry: Jinv[r][x] = d r / d x (Gmsh reference coordinates), stored D x D row-major,
+// and per element face the unit outward normal J^-T n_ref / |J^-T n_ref| (D components) and the face
+// scale sJ/|detJ| = |J^-T n_ref| * fsc, computed in FP64 and rounded once to T.
 template <typename T>
 __global__ void k_geometry(int64_t K, int D, const double* __restrict__ vxyz, T* __restrict__ Jinv,
                            T* __restrict__ fgeom, FaceRef fr, int* __restrict__ err) {
@@ -183,8 +182,8 @@ __global__ void k_geometry(int64_t K, int D, const double* __restrict__ vxyz, T*
     inv[2][1] = (J[0][1] * J[2][0] - J[0][0] * J[2][1]) / det;
     inv[2][2] = (J[0][0] * J[1][1] - J[0][1] * J[1][0]) / det;
   }
-  for (int r = 0; r < 3; ++r)
-    for (int x = 0; x < 3; ++x) Jinv[e * 9 + r * 3 + x] = (T)inv[r][x];
+  for (int r = 0; r < D; ++r)
+    for (int x = 0; x < D; ++x) Jinv[(e * D + r) * D + x] = (T)inv[r][x];
   for (int j = 0; j <= D; ++j) {
     double n[3];
     for (int x = 0; x < 3; ++x) {
@@ -193,8 +192,9 @@ __global__ void k_geometry(int64_t K, int D, const double* __restrict__ vxyz, T*
       n[x] = s;
     }
     double len = sqrt(n[0] * n[0] + n[1] * n[1] + n[2] * n[2]);
-    for (int x = 0; x < 3; ++x) fgeom[(e * (D + 1) + j) * 4 + x] = (T)(n[x] / len);
-    fgeom[(e * (D + 1) + j) * 4 + 3] = (T)(len * fr.fsc[j]);
+    T* const fg = fgeom + (e * (D + 1) + j) * (D + 1);
+    for (int x = 0; x < D; ++x) fg[x] = (T)(n[x] / len);
+    fg[D] = (T)(len * fr.fsc[j]);
   }
 }
 
@@ -310,13 +310,14 @@ void build_geometry(Ctx& c, const double* vxyz_dev) {
 
 namespace {
 template <typename T>
-__global__ void k_scale_geometry(int64_t e0, int64_t n, int NF, double s, T* __restrict__ Jinv,
+__global__ void k_scale_geometry(int64_t e0, int64_t n, int D, double s, T* __restrict__ Jinv,
                                  T* __restrict__ fgeom) {
   int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (i >= n) return;
   int64_t e = e0 + i;
-  for (int c = 0; c < 9; ++c) Jinv[e * 9 + c] = (T)((double)Jinv[e * 9 + c] * s);
-  for (int j = 0; j < NF; ++j) fgeom[(e * NF + j) * 4 + 3] = (T)((double)fgeom[(e * NF + j) * 4 + 3] * s);
+  auto scale = [&](T& v) { v = (T)((double)v * s); };
+  for (int c = 0; c < D * D; ++c) scale(Jinv[e * (D * D) + c]);
+  for (int j = 0; j <= D; ++j) scale(fgeom[(e * (D + 1) + j) * (D + 1) + D]);
 }
 }  // namespace
 
@@ -326,10 +327,10 @@ void scale_geometry(Ctx& c, int64_t e0, int64_t n, double s) {
   if (n <= 0) return;
   unsigned nb = (unsigned)((n + 255) / 256);
   if (c.precision == DGK_FP64)
-    hipLaunchKernelGGL(k_scale_geometry<double>, dim3(nb), dim3(256), 0, c.stream, e0, n, c.Nf, s, (double*)c.Jinv,
+    hipLaunchKernelGGL(k_scale_geometry<double>, dim3(nb), dim3(256), 0, c.stream, e0, n, c.dim, s, (double*)c.Jinv,
                        (double*)c.fgeom);
   else
-    hipLaunchKernelGGL(k_scale_geometry<float>, dim3(nb), dim3(256), 0, c.stream, e0, n, c.Nf, s, (float*)c.Jinv,
+    hipLaunchKernelGGL(k_scale_geometry<float>, dim3(nb), dim3(256), 0, c.stream, e0, n, c.dim, s, (float*)c.Jinv,
                        (float*)c.fgeom);
   DGK_HIP(hipGetLastError());
 }

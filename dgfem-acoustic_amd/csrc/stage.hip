@@ -96,8 +96,8 @@ __global__ __launch_bounds__(kBlock) void k_stage_lds(StageArgs a) {
       sU[q][r] = r < ne * NP ? Vin[q * KN + e0 * NP + r] : (T)0;
     }
     for (int idx = tid; idx < TE * 9; idx += kBlock) {
-      int e = idx / 9, c = idx - e * 9;
-      sG[e][c] = e < ne ? Jinv[(e0 + e) * 9 + c] : (T)0;
+      int e = idx / 9, r = (idx - e * 9) / 3, x = idx % 3;
+      sG[e][r * 3 + x] = e < ne && r < D && x < D ? Jinv[(e0 + e) * (D * D) + r * D + x] : (T)0;
     }
     __syncthreads();
     // outward unit normals and face scale sJ/|detJ| from the inverse Jacobian
@@ -433,7 +433,7 @@ struct MfmaCfg {
   static constexpr int RBP = rb_stride<T>(M::RB > (LES + 3) / 4 ? M::RB : (LES + 3) / 4);
   static constexpr int NSB = 4 * TE * RBP;
   static_assert(LES <= 4 * RBP, "an element's results take the place of its face fluxes");
-  static constexpr size_t kLdsRest = sizeof(T) * (TE * LES + NSB + TE * NF * 4 + TE * 9) +
+  static constexpr size_t kLdsRest = sizeof(T) * (TE * LES + NSB + TE * NF * 4 + TE * D * D) +
                                      sizeof(int) * NF * NPERM * NFP + (LO ? 16 * M::MB * M::NLO * 64 : 0);
   static constexpr size_t kLdsMax = 160 * 1024 - 512;
   // Operator fragments are staged in LDS whenever the whole workgroup footprint fits the 160 KiB
@@ -485,8 +485,13 @@ __global__ __launch_bounds__((MfmaLaunch<T, D, P, SH>::KB), (MfmaLaunch<T, D, P,
   static_assert(ES == D + 1 || ES == 4, "ES: the live field count");
   static_assert(GE * NP * ES % VW == 0, "whole vectors per group");
   constexpr int NE = (GV + GT - 1) / GT;                    // state vectors per thread
-  constexpr int NGEO = (GE * 9 + GT - 1) / GT;              // geometry values per thread
-  constexpr int NFC = (GE * NF * 4 + GT - 1) / GT;          // face geometry values per thread
+  // J^-1 (D x D) and per face the normal's D components and the scale: the geometry is a third of the
+  // bytes that a 2D order 2 stage moves when held as 3 x 3 and 4 per face (us per stage in graph replay,
+  // before -> after: 2D order 2, 980,000 elements, FP64 149.6 -> 143.0, FP32 94.7 -> 91.9; 179,998, FP64,
+  // 28.3 -> 27.7; order 3 FP64, 500,000, 97.3 -> 94.6). LDS keeps four values per face: one vector read.
+  constexpr int GJ = GE * D * D, GF = GE * NF * (D + 1);    // geometry values of a group
+  constexpr int NGEO = (GJ + GT - 1) / GT;                  // per thread
+  constexpr int NFC = (GF + GT - 1) / GT;
   // Face work: TPF threads share one element face, thread kk of them taking the face nodes kk,
   // kk + TPF, ... (NI rounds), so that the face's connectivity, normal and flux coefficients are
   // loaded and formed once per thread and tile, every LDS address is an invariant of the thread plus
@@ -505,7 +510,7 @@ __global__ __launch_bounds__((MfmaLaunch<T, D, P, SH>::KB), (MfmaLaunch<T, D, P,
   constexpr int NSB = C::NSB;
   __shared__ __attribute__((aligned(16))) T sB[NSB];
   __shared__ __attribute__((aligned(32))) T sN[TE * NF * 4];
-  __shared__ T sG[TE * 9];
+  __shared__ __attribute__((aligned(32))) T sG[TE * D * D];
   __shared__ uint32_t sVmap[NF * NPERM * NFP];  // byte offset of the neighbour's node in its element
   constexpr bool kALds = C::kALds;
   constexpr bool kCompact = C::kCompact;
@@ -581,6 +586,12 @@ __global__ __launch_bounds__((MfmaLaunch<T, D, P, SH>::KB), (MfmaLaunch<T, D, P,
   // neighbour traces of tile t+1 are gathered right after tile t's flux phase.
   VT pst[NE];
   T pgeo[NGEO], pfg[NFC];
+  int nof[NFC];  // where a face's values go in LDS: four per face, one vector read
+#pragma unroll
+  for (int t = 0; t < NFC; ++t) {
+    const int i = grp * GF + gtid + t * GT;
+    nof[t] = i / (D + 1) * 4 + i % (D + 1);
+  }
   int2 inc, cnc;
   T iqp[NI][4];
   // value `rel` of an array of `per` values per element, at the tile starting at element e0 (32-bit
@@ -596,11 +607,10 @@ __global__ __launch_bounds__((MfmaLaunch<T, D, P, SH>::KB), (MfmaLaunch<T, D, P,
       if (has_vec(t)) pst[t] = *(const VT*)tile_at(Vin, e0, NP * ES, voff[t]);
 #pragma unroll
     for (int t = 0; t < NGEO; ++t)
-      if (gtid + t * GT < GE * 9) pgeo[t] = *tile_at(Jinv, e0, 9, (uint32_t)(grp * GE * 9 + gtid + t * GT));
+      if (gtid + t * GT < GJ) pgeo[t] = *tile_at(Jinv, e0, D * D, (uint32_t)(grp * GJ + gtid + t * GT));
 #pragma unroll
     for (int t = 0; t < NFC; ++t)
-      if (gtid + t * GT < GE * NF * 4)
-        pfg[t] = *tile_at(Fg, e0, NF * 4, (uint32_t)(grp * GE * NF * 4 + gtid + t * GT));
+      if (gtid + t * GT < GF) pfg[t] = *tile_at(Fg, e0, NF * (D + 1), (uint32_t)(grp * GF + gtid + t * GT));
     inc = make_int2(*tile_at(a.nbr, e0, NF, (uint32_t)fp), *tile_at(a.code, e0, NF, (uint32_t)fp));
   };
   auto gather = [&]() {
@@ -665,10 +675,10 @@ __global__ __launch_bounds__((MfmaLaunch<T, D, P, SH>::KB), (MfmaLaunch<T, D, P,
       if (has_vec(t)) *(VT*)(sU + loff[t]) = pst[t];
 #pragma unroll
     for (int t = 0; t < NGEO; ++t)
-      if (gtid + t * GT < GE * 9) sG[grp * GE * 9 + gtid + t * GT] = pgeo[t];
+      if (gtid + t * GT < GJ) sG[grp * GJ + gtid + t * GT] = pgeo[t];
 #pragma unroll
     for (int t = 0; t < NFC; ++t)
-      if (gtid + t * GT < GE * NF * 4) sN[grp * GE * NF * 4 + gtid + t * GT] = pfg[t];
+      if (gtid + t * GT < GF) sN[nof[t]] = pfg[t];
     // Epilogue operands. pe: u_n (at stage 3 without the compensated solution: W); pa: the accumulator.
     // They are touched once per stage per element, and on large meshes more than the caches hold passes
     // before their next use: their loads and stores carry the non-temporal hint, which leaves the caches
@@ -720,8 +730,8 @@ __global__ __launch_bounds__((MfmaLaunch<T, D, P, SH>::KB), (MfmaLaunch<T, D, P,
     //   fs fl_v = fs A (vne (vm + vp) + (pm + pp)/rho n) + fs H (vm - vp)
     {
       T nf[4];
-      node_fields<4>(sN + fp * 4, nf);
-      const T n[3] = {nf[0], nf[1], nf[2]}, fs = nf[3];
+      node_fields<D == 1 ? 2 : 4>(sN + fp * 4, nf);
+      const T n[3] = {nf[0], D > 1 ? nf[1] : (T)0, D > 2 ? nf[2] : (T)0}, fs = nf[D];
       const bool inter = cnc.x >= 0, refl = cnc.x == -2;
       const T A = fs * ((inter || refl) ? (T)0.5 : (T)0.25);
       const T H = fs * (inter ? (T)0.5 * ((cnc.y >> 16) & 1 ? -c0 : c0) : (refl ? (T)0 : (T)0.25 * c0));
@@ -757,14 +767,19 @@ __global__ __launch_bounds__((MfmaLaunch<T, D, P, SH>::KB), (MfmaLaunch<T, D, P,
     // phase 3: per-lane coefficients Ft_r = alpha_r p + sum_x beta_rx v_x, then the MFMA chain
     T alpha[D], beta[D][3];
     {
-      const T* G = sG + el * 9;
+      T G[D * D];
+      if constexpr (D == 2) node_fields<4>(sG + el * 4, G);
+      else for (int c = 0; c < D * D; ++c) G[c] = sG[el * (D * D) + c];
       for (int r = 0; r < D; ++r) {
-        const T at = G[r * 3 + 0] * v0[0] + G[r * 3 + 1] * v0[1] + G[r * 3 + 2] * v0[2];
+        T at = G[r * D] * v0[0];
+        for (int x = 1; x < D; ++x) at += G[r * D + x] * v0[x];
         if (q == 0) {
           alpha[r] = at;
-          for (int x = 0; x < 3; ++x) beta[r][x] = rc2 * G[r * 3 + x];
+          for (int x = 0; x < 3; ++x) beta[r][x] = x < D ? rc2 * G[r * D + x] : (T)0;
         } else {
-          alpha[r] = G[r * 3 + (q - 1)] * irho;
+          T gq = 0;
+          for (int x = 0; x < D; ++x) gq = x == q - 1 ? G[r * D + x] : gq;
+          alpha[r] = gq * irho;
           for (int x = 0; x < 3; ++x) beta[r][x] = (x == q - 1) ? at : (T)0;
         }
       }
