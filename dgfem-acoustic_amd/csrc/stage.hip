@@ -518,17 +518,31 @@ __global__ __launch_bounds__((MfmaLaunch<T, D, P, SH>::KB), (MfmaLaunch<T, D, P,
   __shared__ bf16x8 sAlo[LO ? MB * NLO * 64 : 1];
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  // wave = rg * (TE/4) + element group; lane group g, column col = 4 * (element in group) + field q
-  const int rg = RG > 1 ? wave / (TE / 4) : 0;
-  const int we = wave % (TE / 4), grp = we / GW, gtid = (rg * GW + we % GW) * 64 + lane;
+  // wave = RG * (4 elements) + row group: consecutive waves sit on different SIMDs, so each SIMD runs one
+  // wave of every element group; lane group g, column col = 4 * (element in group) + field q
+  const int rg = wave % RG, we = wave / RG, grp = we / GW, gtid = (rg * GW + we % GW) * 64 + lane;
   const int g = lane >> 4, col = lane & 15, el = we * 4 + (col >> 2), q = col & 3;
   // a group's results take the place of its face fluxes, element el at el * LES of sR
   T* const sR = sB + grp * GE * (4 * RB - LES);
   // orders the group's LDS accesses: within one wave LDS works in program order and only the compiler
-  // has to keep it
+  // has to keep it. The row split's groups of several waves meet at a counter of their own in LDS: with
+  // the workgroup's barrier both groups did their fluxes together and left the matrix cores idle
+  // meanwhile (half of the time). All waves of a group walk the same tiles and so arrive at the same
+  // meetings; none leaves early. us per stage (graph replay), barrier -> counters: 3D order 5 FP64,
+  // 82,944 elements, 283 -> 267; 7722, 31.2 -> 30.5.
+  __shared__ uint32_t sMet[TE / GE];
+  uint32_t met = 0;  // arrivals in the group at its next meeting
+  if (GT > 64 && GT < kBlock && tid < TE / GE) sMet[tid] = 0;  // the start-up's barrier comes before the first meeting
   auto sync = [&]() {
-    if constexpr (GT > 64) {
+    if constexpr (GT == kBlock) {
       __syncthreads();
+    } else if constexpr (GT > 64) {
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+      met += GT / 64;
+      if (lane == 0) __hip_atomic_fetch_add(&sMet[grp], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      while ((int)(__hip_atomic_load(&sMet[grp], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) - met) < 0) {
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
     } else {
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
       __builtin_amdgcn_wave_barrier();
@@ -835,17 +849,18 @@ __global__ __launch_bounds__((MfmaLaunch<T, D, P, SH>::KB), (MfmaLaunch<T, D, P,
         for (int c = 1; c < ES; ++c) v = fma(beta[r][c - 1], f[c], v);
         return v;
       };
-      if constexpr (kALds && !(sizeof(T) == 8 && D == 3)) {
+      if constexpr (kALds && !(sizeof(T) == 8 && D == 3 && RG == 1)) {
         // Software pipeline, one region of the schedule per k-step: the first MFMA of k-step s is
         // issued, then (in its shadow) the LDS reads of the operator and face values PF k-steps
         // ahead and of the next node group, and the B value of k-step s+1, then the other MFMAs of
         // k-step s. The fences keep the compiler from sinking the reads back to their uses, where
-        // every k-step waits for the LDS latency. FP64 holds one k-step ahead (its registers), and in
-        // 3D none: order 3 would spill 49 registers (105 -> 261 us per stage, 196,608 elements), order 5
-        // loses 2%. us per stage in graph replay, unrolled loop -> pipeline: 2D order 3 FP64, 500,000
-        // elements, 100.7 -> 96.5; order 4, 320,000, 88.5 -> 82.4; FP32 2D order 2, 980,000, 97.2 -> 95.0;
-        // 3D order 5, 82,944, 118 -> 113; order 3, 196,608, 66.5 -> 65.5.
-        constexpr int PF = sizeof(T) == 4 ? 4 : 1, NS = PF + 1;
+        // every k-step waits for the LDS latency. FP64 holds one k-step ahead (its registers; four in the
+        // row split, whose waves have one row block each) and in 3D without the row split none: order 3
+        // would spill 49 registers (105 -> 261 us per stage, 196,608 elements). us per stage in graph
+        // replay, unrolled loop -> pipeline: 2D order 3 FP64, 500,000 elements, 100.7 -> 96.5; order 4,
+        // 320,000, 88.5 -> 82.4; 3D order 5 FP64, 82,944, 267 -> 264; FP32 2D order 2, 980,000, 97.2 ->
+        // 95.0; 3D order 5, 82,944, 118 -> 113; order 3, 196,608, 66.5 -> 65.5.
+        constexpr int PF = sizeof(T) == 4 || RG > 1 ? 4 : 1, NS = PF + 1;
         T fn[2][4], af[NS][MBW ? MBW : 1], tf[NS][NT4 ? NT4 : 1], ff[NS];
         auto load_op = [&](const int s) {
 #pragma unroll
