@@ -8,6 +8,7 @@
 #include <cmath>
 #include <cstring>
 #include <exception>
+#include <memory>
 #include <unordered_map>
 
 #include "dgk_internal.hpp"
@@ -237,7 +238,8 @@ void create_impl(Ctx& c, const dgk_mesh* m, const dgk_phys* ph, const dgk_opts* 
   c.rho0 = ph->rho0;
   for (int k = 0; k < 3; ++k) c.v0[k] = ph->v0[k];
   c.fc = (c.dim == 3 && c.p != 1) ? -1 : 1;  // src/Mesh.cpp:210-211
-  RefElem R = make_ref_elem(c.dim, c.p);
+  c.ref = std::make_shared<const RefElem>(make_ref_elem(c.dim, c.p));
+  const RefElem& R = *c.ref;
   c.Np = R.Np;
   c.Nf = R.Nf;
   c.Nfp = R.Nfp;
@@ -445,9 +447,9 @@ double bary_score(int d, int Np, const double* node_xyz, int64_t e, const double
 // of about K cells, the one whose smallest barycentric coordinate of the point is largest. Returns the
 // elements; w receives, per point, the element's Lagrange basis at the point (pressure = sum_n w[n]
 // p[e*Np+n]).
-// The points are binned, not the elements: one pass over the vertices on several threads finds the mesh's
+// The points are binned, not the elements: one pass over the vertices finds the mesh's
 // extent and the few elements whose (slightly grown) box holds a point; an element that accepts a point
-// (coordinate >= -1e-6) is among them. 196,608 elements, 16 points: 24.4 -> 2.8 ms.
+// (coordinate >= -1e-6) is among them. 196,608 elements, 16 points: 24.4 -> 4.2 ms.
 std::vector<int64_t> locate_points(const RefElem& R, const double* node_xyz, int64_t K, int n, const double* xyz,
                                    std::vector<double>& w) {
   const int d = R.dim, Np = R.Np;
@@ -480,15 +482,6 @@ std::vector<int64_t> locate_points(const RefElem& R, const double* node_xyz, int
     std::vector<int> fill(pstart.begin(), pstart.end() - 1);
     for (int p = 0; p < n; ++p) pitem[fill[pof(p)]++] = p;
   }
-  struct Hit {
-    int p;
-    int64_t e;
-  };
-  struct Found {
-    double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300};
-    std::vector<Hit> hits;
-    std::exception_ptr err;
-  };
   auto bounds = [&](int64_t e, double a[3], double b[3]) {
     const double* X = node_xyz + (size_t)e * Np * 3;
     for (int c = 0; c < 3; ++c) a[c] = b[c] = X[c];
@@ -498,47 +491,38 @@ std::vector<int64_t> locate_points(const RefElem& R, const double* node_xyz, int
         b[c] = std::max(b[c], X[3 * v + c]);
       }
   };
-  std::vector<Found> found(8);
-  parallel_ranges(K, 16384, [&](int t, int64_t e0, int64_t e1) {
-    Found& f = found[t];
-    try {
-      for (int64_t e = e0; e < e1; ++e) {
-        double a[3], b[3];
-        bounds(e, a, b);
-        bool out_of_reach = false;
-        for (int c = 0; c < 3; ++c) {
-          f.lo[c] = std::min(f.lo[c], a[c]);
-          f.hi[c] = std::max(f.hi[c], b[c]);
-          if (c >= d) continue;
-          const double grow = 1e-4 * (b[c] - a[c]) + 1e-8 * (1 + std::fabs(a[c]) + std::fabs(b[c]));
-          a[c] -= grow;
-          b[c] += grow;
-          out_of_reach |= !(b[c] >= plo[c] && a[c] <= phi_[c]);
-        }
-        if (out_of_reach) continue;
-        for (int i = pcell(0, a[0]), i1 = pcell(0, b[0]); i <= i1; ++i)
-          for (int j = d > 1 ? pcell(1, a[1]) : 0, j1 = d > 1 ? pcell(1, b[1]) : 0; j <= j1; ++j)
-            for (int k = d > 2 ? pcell(2, a[2]) : 0, k1 = d > 2 ? pcell(2, b[2]) : 0; k <= k1; ++k)
-              for (int m = pstart[pindex(i, j, k)]; m < pstart[pindex(i, j, k) + 1]; ++m) {
-                const double* x = xyz + 3 * (size_t)pitem[m];
-                bool in = true;
-                for (int c = 0; c < d; ++c) in &= x[c] >= a[c] && x[c] <= b[c];
-                if (in) f.hits.push_back({pitem[m], e});
-              }
-      }
-    } catch (...) {
-      f.err = std::current_exception();
-    }
-  });
+  // One thread: helpers saved 1-2 ms of a 196,608-element mesh's 4 on a quiet machine, but the caller's other
+  // threads (an OpenMP pool after a loop) may spin on every core, and a helper then starts, or is joined,
+  // at the end of a time slice, 4 ms later.
   double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300};
-  std::vector<std::vector<int64_t>> cand(n);
-  for (auto& f : found) {  // ranges in element order, so every point's candidates ascend
-    if (f.err) std::rethrow_exception(f.err);
+  std::vector<std::vector<int64_t>> cand(n);  // the elements whose bounds hold a point, ascending
+  for (int64_t e = 0; e < K; ++e) {
+    // the vertices of an element to come (they lead its Np nodes)
+    const double* ahead = node_xyz + (size_t)std::min(e + 16, K - 1) * Np * 3;
+    __builtin_prefetch(ahead);
+    __builtin_prefetch(ahead + 3 * d + 2);
+    double a[3], b[3];
+    bounds(e, a, b);
+    bool out_of_reach = false;
     for (int c = 0; c < 3; ++c) {
-      lo[c] = std::min(lo[c], f.lo[c]);
-      hi[c] = std::max(hi[c], f.hi[c]);
+      lo[c] = std::min(lo[c], a[c]);
+      hi[c] = std::max(hi[c], b[c]);
+      if (c >= d) continue;
+      const double grow = 1e-4 * (b[c] - a[c]) + 1e-8 * (1 + std::fabs(a[c]) + std::fabs(b[c]));
+      a[c] -= grow;
+      b[c] += grow;
+      out_of_reach |= !(b[c] >= plo[c] && a[c] <= phi_[c]);
     }
-    for (auto& h : f.hits) cand[h.p].push_back(h.e);
+    if (out_of_reach) continue;
+    for (int i = pcell(0, a[0]), i1 = pcell(0, b[0]); i <= i1; ++i)
+      for (int j = d > 1 ? pcell(1, a[1]) : 0, j1 = d > 1 ? pcell(1, b[1]) : 0; j <= j1; ++j)
+        for (int k = d > 2 ? pcell(2, a[2]) : 0, k1 = d > 2 ? pcell(2, b[2]) : 0; k <= k1; ++k)
+          for (int m = pstart[pindex(i, j, k)]; m < pstart[pindex(i, j, k) + 1]; ++m) {
+            const double* x = xyz + 3 * (size_t)pitem[m];
+            bool in = true;
+            for (int c = 0; c < d; ++c) in &= x[c] >= a[c] && x[c] <= b[c];
+            if (in) cand[pitem[m]].push_back(e);
+          }
   }
   int g[3] = {1, 1, 1};
   const int gd = (int)std::max(1.0, std::floor(std::pow((double)K, 1.0 / d)));
@@ -583,16 +567,7 @@ std::vector<int64_t> locate_points(const RefElem& R, const double* node_xyz, int
     for (int k = 0; k < Np; ++k) w[(size_t)p * Np + k] = (double)phi[k];
     out[p] = best;
   };
-  std::vector<std::exception_ptr> errs(8);
-  parallel_ranges(n, 8, [&](int t, int64_t p0, int64_t p1) {
-    try {
-      for (int64_t p = p0; p < p1; ++p) locate((int)p);
-    } catch (...) {
-      errs[t] = std::current_exception();
-    }
-  });
-  for (auto& e : errs)
-    if (e) std::rethrow_exception(e);
+  for (int p = 0; p < n; ++p) locate(p);
   for (int p = 0; p < n; ++p)
     if (out[p] < 0) throw InvalidArg("receiver point " + std::to_string(p) + " lies outside the mesh");
   return out;
@@ -928,7 +903,7 @@ dgk_status dgk_set_sources(dgk_ctx* c, int n, const double* src, const double* n
 dgk_status dgk_set_receivers(dgk_ctx* c, int n, const double* xyz, const double* node_xyz, int capacity) {
   if (!c || n < 0 || (n > 0 && (!xyz || !node_xyz))) return fail(c, DGK_ERR_INVALID, "bad receiver arguments");
   return guarded(c, [&] {
-    RefElem R = make_ref_elem(c->dim, c->p);
+    const RefElem& R = *c->ref;
     std::vector<double> w;
     std::vector<int64_t> elem = locate_points(R, node_xyz, c->K, n, xyz, w);
     install_receivers(*c, elem, w, capacity);
@@ -1417,7 +1392,7 @@ dgk_status dgk_batch_set_receivers(dgk_batch* b, int sim, int n, const double* x
     std::vector<size_t> col0(nm, 0);
     for (size_t k = 1; k < nm; ++k) col0[k] = col0[k - 1] + G.rel[k - 1].size();
     const size_t nold = c.rec.n;
-    dgk::RefElem R = dgk::make_ref_elem(c.dim, c.p);
+    const dgk::RefElem& R = *c.ref;
     std::vector<double> wt;
     std::vector<int64_t> el = dgk::locate_points(R, node_xyz, b->K[sim], n, xyz, wt);
     G.rel[w.second] = el;

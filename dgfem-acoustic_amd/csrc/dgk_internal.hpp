@@ -4,6 +4,7 @@
 
 #include <cstdint>
 #include <map>
+#include <memory>
 #include <stdexcept>
 #include <string>
 #include <vector>
@@ -95,7 +96,10 @@ struct StageArgs {
   int addr64;      // 1: 64-bit per-tile bases even when every array fits 32-bit offsets
 };
 
+struct RefElem;
+
 struct Ctx {
+  std::shared_ptr<const RefElem> ref;  // the reference element of (dim, p)
   int dim = 0, p = 0, Np = 0, Nf = 0, Nfp = 0, nperm = 1;
   int64_t K = 0, F = 0, Fb = 0;
   int64_t Kpad = 0, PS = 0;  // elements padded to kTilePad, field plane stride (values)
@@ -205,7 +209,6 @@ struct Tuned {
   int variant = 0, grid_pct = 100, tile_order = 0, tile_shape = 0;
 };
 bool find_tuning(int dim, int p, int precision, Tuned* t);
-struct RefElem;
 std::vector<int64_t> locate_points(const RefElem& R, const double* node_xyz, int64_t K, int n, const double* xyz,
                                    std::vector<double>& w);
 void install_receivers(Ctx& c, const std::vector<int64_t>& elem, const std::vector<double>& w, int cap);

@@ -11,28 +11,9 @@
 #include <cstring>
 #include <exception>
 #include <mutex>
-#include <system_error>
-#include <thread>
 #include <vector>
 
 namespace dgk {
-
-// fn(i) for i in [0, n) on up to 8 threads, in contiguous ranges; fn must not throw.
-template <class F>
-void parallel_ranges(int64_t n, int64_t grain, F&& fn /* (thread, begin, end) */) {
-  const int64_t most = std::min<int64_t>(8, std::max(1u, std::thread::hardware_concurrency()));
-  const int nt = (int)std::max<int64_t>(1, std::min(most, n / std::max<int64_t>(1, grain)));
-  std::vector<std::thread> th;
-  for (int t = 1; t < nt; ++t) {
-    try {
-      th.emplace_back([&, t] { fn(t, n * t / nt, n * (t + 1) / nt); });
-    } catch (const std::system_error&) {  // no thread to be had: this one does the work
-      fn(t, n * t / nt, n * (t + 1) / nt);
-    }
-  }
-  fn(0, 0, n / nt);
-  for (auto& x : th) x.join();
-}
 
 // Page-locked slabs of kSlabBytes, shared by all contexts and threads of the process: a call takes one
 // for itself and gives it back; at most kSlabsKept wait for the next call, and the last user to leave

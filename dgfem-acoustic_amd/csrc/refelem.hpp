@@ -248,12 +248,12 @@ struct RefElem {
     modal_eval(modal, x, v.data(), reinterpret_cast<ld(*)[3]>(g.data()));
     for (int n = 0; n < Np; ++n) {
       ld s = 0, gs[3] = {0, 0, 0};
-      for (int m = 0; m < Np; ++m) {
-        s += C[n * Np + m] * v[m];
-        for (int b = 0; b < 3; ++b) gs[b] += C[n * Np + m] * g[m][b];
-      }
+      for (int m = 0; m < Np; ++m) s += C[n * Np + m] * v[m];
       phi[n] = s;
-      if (dphi) for (int b = 0; b < 3; ++b) dphi[n][b] = gs[b];
+      if (!dphi) continue;
+      for (int m = 0; m < Np; ++m)
+        for (int b = 0; b < 3; ++b) gs[b] += C[n * Np + m] * g[m][b];
+      for (int b = 0; b < 3; ++b) dphi[n][b] = gs[b];
     }
   }
 };
