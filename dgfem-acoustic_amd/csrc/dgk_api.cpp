@@ -759,9 +759,9 @@ namespace {
 // dgk_rhs 125 -> 57 us). Half a slab in, half out.
 constexpr size_t kDirectBytes = (size_t)1 << 20;
 static_assert(kDirectBytes <= Slabs::kSlabBytes / 2, "a state in and a state out of one slab");
-double* slab_in(Slab& s) { return (double*)s.p; }
-double* slab_out(Slab& s) { return (double*)(s.p + Slabs::kSlabBytes / 2); }
-bool direct(const Slab& s, int64_t n) { return s.p && 4 * (size_t)n * sizeof(double) <= kDirectBytes; }
+double* slab_in(Slab& s) { return (double*)s.data(); }
+double* slab_out(Slab& s) { return (double*)(s.data() + Slabs::kSlabBytes / 2); }
+bool direct(Slab& s, int64_t n) { return 4 * (size_t)n * sizeof(double) <= kDirectBytes && s.data(); }
 
 // Host u[4][n] (FP64) -> nodes [off, off+n) of a device state buffer in the state precision and layout.
 // Asynchronous: u (or the slab) is read until the stream is synchronised.
@@ -785,7 +785,7 @@ void upload_planes(Ctx& c, const double* u, void* dst, int64_t off, int64_t n, S
 void download_planes(Ctx& c, const void* src, double* u, int64_t off, int64_t n, Slab& slab) {
   const uint16_t* lo = src == c.U && c.comp ? c.Ulo : nullptr;
   const int live = c.es > 1 ? c.es : 4;
-  if (direct(slab, n) && c.es > 1) {
+  if (c.es > 1 && direct(slab, n)) {
     state_to_f64(c, src, lo, slab_out(slab), n, off, n);
     DGK_HIP(hipStreamSynchronize(c.stream));
     memcpy(u, slab_out(slab), live * n * sizeof(double));
@@ -799,7 +799,7 @@ void download_planes(Ctx& c, const void* src, double* u, int64_t off, int64_t n,
     std::vector<Piece> p;
     for (int q = 0; q < live; ++q)
       p.push_back({(const char*)(s + q * c.PS), (char*)(u + q * n), n * sizeof(double)});
-    DGK_HIP(download(p, c.stream));
+    DGK_HIP(download(p, c.stream, slab));
   }
   std::fill(u + live * n, u + 4 * n, 0.0);
 }

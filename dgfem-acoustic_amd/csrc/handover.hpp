@@ -79,22 +79,30 @@ struct SlabUser {
   SlabUser& operator=(const SlabUser&) = delete;
 };
 
-// One slab for the length of a call (null when none is to be had). Work on stream s that uses it is
-// over when the call ends in the ordinary way; when an exception ends it, it is waited for here.
-struct Slab {
-  char* p;
-  explicit Slab(hipStream_t s) : p((char*)Slabs::get().take()), s_(s), unwinding_(std::uncaught_exceptions()) {}
+// At most one slab for the length of a call, taken where data() is first asked for (null when none is to
+// be had): a call that needs none takes none. Work on stream s that uses it is over when the call ends in
+// the ordinary way; when an exception ends it, it is waited for here.
+class Slab {
+ public:
+  explicit Slab(hipStream_t s) : s_(s), unwinding_(std::uncaught_exceptions()) {}
   ~Slab() {
-    if (!p) return;
+    if (!p_) return;
     if (std::uncaught_exceptions() > unwinding_) (void)hipStreamSynchronize(s_);
-    Slabs::get().give(p);
+    Slabs::get().give(p_);
   }
   Slab(const Slab&) = delete;
   Slab& operator=(const Slab&) = delete;
+  char* data() {
+    if (!asked_) p_ = (char*)Slabs::get().take();
+    asked_ = true;
+    return p_;
+  }
 
  private:
   hipStream_t s_;
   int unwinding_;
+  bool asked_ = false;
+  char* p_ = nullptr;
 };
 
 // A piece of a transfer: `bytes` from device memory to host memory.
@@ -104,26 +112,26 @@ struct Piece {
   size_t bytes;
 };
 
-// Copies device pieces to host memory through a slab in slots of 2 MB: while slots are in transfer, this
-// thread copies out the one that has landed. Blocks until everything is in place. The thread polls: one
-// that sleeps gets its core back only at the end of a time slice when the caller's other threads (an
-// OpenMP pool after a loop) spin on all of them, 4 ms a call; for the same reason the copying has no
-// helper threads, which took 3 of 126 MB's 9.5 ms off on a quiet machine and cost 3 ms a call beside
-// spinning ones.
-inline hipError_t download(const std::vector<Piece>& pieces, hipStream_t s) {
+// Copies device pieces to host memory through the call's slab in slots of 2 MB: while slots are in transfer,
+// this thread copies out the one that has landed. Blocks until everything is in place. What the slab held
+// is overwritten, in the order of stream s. The thread polls: one that sleeps gets its core back only at the
+// end of a time slice when the caller's other threads (an OpenMP pool after a loop) spin on all of them, 4 ms
+// a call; for the same reason the copying has no helper threads, which took 3 of 126 MB's 9.5 ms off on a
+// quiet machine and cost 3 ms a call beside spinning ones.
+inline hipError_t download(const std::vector<Piece>& pieces, hipStream_t s, Slab& slab) {
   constexpr size_t kSlot = (size_t)2 << 20, kSlots = Slabs::kSlabBytes / kSlot;
   std::vector<Piece> part;
   for (auto& q : pieces)
     for (size_t o = 0; o < q.bytes; o += kSlot)
       part.push_back({q.dev + o, q.host + o, std::min(kSlot, q.bytes - o)});
   const size_t n = part.size();
-  Slab slab(s);
-  if (!slab.p || n < 2) {
-    for (auto& q : pieces) {
-      const hipError_t e = hipMemcpyAsync(q.host, q.dev, q.bytes, hipMemcpyDeviceToHost, s);
-      if (e != hipSuccess) return e;
-    }
-    return hipStreamSynchronize(s);
+  char* const buf = n < 2 ? nullptr : slab.data();
+  if (!buf) {
+    hipError_t e = hipSuccess;
+    for (size_t i = 0; i < pieces.size() && e == hipSuccess; ++i)
+      e = hipMemcpyAsync(pieces[i].host, pieces[i].dev, pieces[i].bytes, hipMemcpyDeviceToHost, s);
+    const hipError_t w = hipStreamSynchronize(s);  // also after an error: the host memory is the caller's
+    return e != hipSuccess ? e : w;
   }
   hipEvent_t ev[kSlots];
   size_t nev = 0;
@@ -131,7 +139,7 @@ inline hipError_t download(const std::vector<Piece>& pieces, hipStream_t s) {
   for (; nev < std::min(n, kSlots); ++nev)
     if ((err = hipEventCreateWithFlags(&ev[nev], hipEventDisableTiming)) != hipSuccess) break;
   auto start = [&](size_t k) {
-    hipError_t e = hipMemcpyAsync(slab.p + (k % kSlots) * kSlot, part[k].dev, part[k].bytes, hipMemcpyDeviceToHost, s);
+    hipError_t e = hipMemcpyAsync(buf + (k % kSlots) * kSlot, part[k].dev, part[k].bytes, hipMemcpyDeviceToHost, s);
     return e == hipSuccess ? hipEventRecord(ev[k % kSlots], s) : e;
   };
   for (size_t k = 0; k < std::min(n, kSlots) && err == hipSuccess; ++k) err = start(k);
@@ -139,7 +147,7 @@ inline hipError_t download(const std::vector<Piece>& pieces, hipStream_t s) {
     while ((err = hipEventQuery(ev[k % kSlots])) == hipErrorNotReady) {
     }
     if (err != hipSuccess) break;
-    memcpy(part[k].host, slab.p + (k % kSlots) * kSlot, part[k].bytes);
+    memcpy(part[k].host, buf + (k % kSlots) * kSlot, part[k].bytes);
     if (k + kSlots < n) err = start(k + kSlots);
   }
   if (err != hipSuccess) (void)hipStreamSynchronize(s);  // no transfer may outlive the slab's loan

@@ -808,22 +808,22 @@ dgs_status dgs_forward(dgs_net* n, int rows, const float* x, float* y) {
       b.hl = &n->h;
       b.prel = &n->pre;
       b.y = n->y;
-      if (slab.p && xbytes <= half) {
-        memcpy(slab.p, x + (size_t)r0 * in, xbytes);
-        b.x = (const float*)slab.p;
+      if (xbytes <= half && slab.data()) {
+        memcpy(slab.data(), x + (size_t)r0 * in, xbytes);
+        b.x = (const float*)slab.data();
       } else {
         DGS_HIP(hipMemcpyAsync(n->x, x + (size_t)r0 * in, xbytes, hipMemcpyHostToDevice, n->s));
         b.x = n->x;
       }
-      const bool direct = slab.p && ybytes <= most;
-      if (direct) b.y = (float*)(slab.p + half);
+      const bool direct = ybytes <= most && slab.data();
+      if (direct) b.y = (float*)(slab.data() + half);
       dgs::forward(*n, mp, b);
       float* to = y + (size_t)r0 * No;
       if (direct) {
         DGS_HIP(hipStreamSynchronize(n->s));
         memcpy(to, b.y, ybytes);
       } else {
-        DGS_HIP(dgk::download({{(const char*)n->y, (char*)to, ybytes}}, n->s));
+        DGS_HIP(dgk::download({{(const char*)n->y, (char*)to, ybytes}}, n->s, slab));
       }
     }
   });
