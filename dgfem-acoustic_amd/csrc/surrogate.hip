@@ -797,6 +797,7 @@ dgs_status dgs_forward(dgs_net* n, int rows, const float* x, float* y) {
     // of it each), without copy commands (100 rows, 2048 outputs: 124 -> 78 us); otherwise the slab only
     // carries the inputs
     constexpr size_t half = dgk::Slabs::kSlabBytes / 2, most = (size_t)2 << 20;
+    static_assert(most <= half, "inputs and outputs of a pass in one slab");
     dgk::Slab slab(n->s);
     for (int r0 = 0; r0 < rows; r0 += mb) {
       const int m = std::min(mb, rows - r0);

@@ -10,6 +10,7 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 RUNTIME = r"""
 #include "handover.hpp"
+#include <atomic>
 #include <cassert>
 #include <cstdio>
 #include <cstdlib>
@@ -112,3 +113,28 @@ def test_download_that_fails_waits_for_what_is_under_way(tmp_path, at, no_memory
     setup = f"copies = 0; fail_copy = {at}; no_memory = {'true' if no_memory else 'false'};"
     run(tmp_path, DOWNLOAD.replace("SETUP", setup).replace(
         "CHECK", "assert(copies > fail_copy ? e == hipErrorUnknown : e == hipSuccess);"))
+
+
+def test_contexts_one_at_a_time_page_lock_once(tmp_path):
+    run(tmp_path, """
+  for (int i = 0; i < 10; ++i) { SlabUser u; Slab s(nullptr); assert(s.data()); }
+  assert(allocs == 1 && most_locked <= (size_t)4 << 20);
+""")
+
+
+def test_the_pool_is_bounded(tmp_path):
+    """Eight threads with a slab each: a few wait for the next calls, one when the last context has gone."""
+    run(tmp_path, """
+  {
+    SlabUser u;
+    std::vector<std::thread> t;
+    std::atomic<int> in{0};
+    for (int i = 0; i < 8; ++i)
+      t.emplace_back([&] { SlabUser v; Slab s(nullptr); assert(s.data()); for (++in; in < 8;) std::this_thread::yield(); });
+    for (auto& x : t) x.join();
+    assert(allocs == 8 && locked.size() == Slabs::kSlabsKept);
+    { Slab a(nullptr), b(nullptr); assert(a.data() != b.data()); }
+    assert(allocs == 8);
+  }
+  assert(locked.size() == 1 && frees == 7);
+""")
