@@ -287,9 +287,10 @@ __global__ __launch_bounds__(256) void k_gemm_large(GemmArgs g) {
 }
 
 // z[r][f] = sin(2 pi B_f . x_r), z[r][F + f] = cos(2 pi B_f . x_r), rounded to BF16.
-// Row r is taken from row idx[r] (when given) or min(r, m - 1) of x.
+// Row r is taken from row idx[r] (when given) or min(r, m - 1) of x, and kept in row r of `keep` (when
+// given).
 __global__ void k_features(int n, int m, int in, int F, const int* __restrict__ idx, const float* __restrict__ x,
-                           const float* __restrict__ Bm, uint16_t* __restrict__ z) {
+                           const float* __restrict__ Bm, uint16_t* __restrict__ z, float* __restrict__ keep) {
   const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (i >= (int64_t)n * F) return;
   const int r = (int)(i / F), f = (int)(i % F);
@@ -299,6 +300,8 @@ __global__ void k_features(int n, int m, int in, int F, const int* __restrict__ 
   a *= 6.283185307179586f;
   z[(int64_t)r * 2 * F + f] = f2bf(sinf(a));
   z[(int64_t)r * 2 * F + F + f] = f2bf(cosf(a));
+  if (keep)
+    for (int d = f; d < in; d += F) keep[(int64_t)r * in + d] = x[xr * in + d];
 }
 
 // Relative squared error per sample: loss_r = w_r sum_j (y - t)^2, w_r = 1 / (n |t_r|^2);
@@ -438,7 +441,7 @@ struct Net {
   float* Bm = nullptr;  // Fourier matrix F x in
   int64_t adam_t = 0;
   // per-batch buffers (max_batch rows)
-  float *x = nullptr, *t = nullptr, *w = nullptr, *y = nullptr, *loss_row = nullptr;
+  float *x = nullptr, *t = nullptr, *w = nullptr, *y = nullptr, *loss_row = nullptr;  // x: the last pass's rows
   uint16_t* z = nullptr;
   std::vector<uint16_t*> h;  // BF16 activations of hidden layers
   std::vector<float*> pre;   // FP32 pre-activations of hidden layers
@@ -513,6 +516,7 @@ struct Pass {
   const float* x;
   int m;                       // rows of x and y
   const int* idx = nullptr;
+  float* keep = nullptr;       // the rows of the pass stay here (Net::x, what dgs_forward_timed runs on)
   uint16_t* z;
   uint16_t* h[2];  // hidden layer l writes h[l % 2] (when not per layer)
   const std::vector<uint16_t*>* hl = nullptr;  // per-layer buffers (training keeps them for backward)
@@ -575,7 +579,7 @@ void forward(Net& n, int rows, const Pass& b) {
   const int F = n.cfg.n_freq, in = n.cfg.in_dim;
   const int64_t tot = (int64_t)rows * F;
   hipLaunchKernelGGL(k_features, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, n.s, rows, b.m, in, F, b.idx, b.x,
-                     n.Bm, b.z);
+                     n.Bm, b.z, b.keep);
   DGS_HIP(hipGetLastError());
   const uint16_t* a = b.z;
   for (int l = 0; l < n.L; ++l) {
@@ -608,6 +612,7 @@ void forward(Net& n, int rows, const int* idx = nullptr) {
   b.x = idx ? n.X : n.x;
   b.m = rows;
   b.idx = idx;
+  if (idx) b.keep = n.x;
   b.z = n.z;
   b.hl = &n.h;
   b.prel = &n.pre;
@@ -726,6 +731,7 @@ void create_impl(Net& n, const dgs_config* c) {
   for (auto& v : hb) v = (float)(k.freq_sigma * nd(rng));
   DGS_HIP(hipMemcpy(n.P, hp.data(), hp.size() * sizeof(float), hipMemcpyHostToDevice));
   DGS_HIP(hipMemcpy(n.Bm, hb.data(), hb.size() * sizeof(float), hipMemcpyHostToDevice));
+  DGS_HIP(hipMemset(n.x, 0, (size_t)mb * k.in_dim * sizeof(float)));
   DGS_HIP(hipMemset(n.Am, 0, n.nparam * sizeof(float)));
   DGS_HIP(hipMemset(n.Av, 0, n.nparam * sizeof(float)));
   DGS_HIP(hipMemset(n.G, 0, n.nparam * sizeof(float)));
@@ -812,6 +818,7 @@ dgs_status dgs_forward(dgs_net* n, int rows, const float* x, float* y) {
       if (xbytes <= half && slab.data()) {
         memcpy(slab.data(), x + (size_t)r0 * in, xbytes);
         b.x = (const float*)slab.data();
+        b.keep = n->x;
       } else {
         DGS_HIP(hipMemcpyAsync(n->x, x + (size_t)r0 * in, xbytes, hipMemcpyHostToDevice, n->s));
         b.x = n->x;

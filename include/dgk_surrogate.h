@@ -51,7 +51,8 @@ dgs_status dgs_forward(dgs_net* net, int rows, const float* x, float* y);
  * fit is rejected with DGS_ERR_INVALID). Ordered on the network's stream and synchronous like dgs_forward. Calls
  * that overlap on one GPU share that array and race. */
 dgs_status dgs_forward_noalloc(dgs_net* net, int rows, const float* x, float* y);
-/* average device time of `reps` forward passes over `rows` rows already on the device */
+/* average device time of `reps` forward passes over `rows` rows already on the device: those of the last
+ * pass of dgs_forward, dgs_gradients or dgs_train (zero where there was none) */
 dgs_status dgs_forward_timed(dgs_net* net, int rows, int reps, double* ms_per_rep);
 /* one forward + backward without update: loss = sum_r w[r] |y_r - t_r|^2 and its gradient
  * (num_params floats, may be NULL); rows a multiple of 64 up to max_batch */
