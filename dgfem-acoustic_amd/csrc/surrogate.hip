@@ -545,9 +545,10 @@ unsigned char* scratch_base(int dev) {
 
 size_t aligned256(size_t bytes) { return (bytes + 255) / 256 * 256; }
 
-// Layout of one forward pass of mp rows in the scratch array (256-byte aligned pieces: features and
-// two layers' activations; inputs and outputs stay in the caller's memory); returns the bytes needed.
-size_t scratch_layout(const Net& n, int mp, unsigned char* base, Pass* b) {
+// Layout of one forward pass of mp rows in the scratch array (256-byte aligned pieces: features, two
+// layers' activations and, with own_y, the outputs, which otherwise go to the caller's memory; inputs stay
+// there); returns the bytes needed.
+size_t scratch_layout(const Net& n, int mp, bool own_y, unsigned char* base, Pass* b) {
   const dgs_config& k = n.cfg;
   const size_t z = aligned256((size_t)mp * 2 * k.n_freq * sizeof(uint16_t));
   const size_t h = aligned256((size_t)mp * k.width * sizeof(uint16_t));
@@ -555,18 +556,31 @@ size_t scratch_layout(const Net& n, int mp, unsigned char* base, Pass* b) {
     b->z = (uint16_t*)base;
     b->h[0] = (uint16_t*)(base + z);
     b->h[1] = (uint16_t*)(base + z + h);
+    if (own_y) b->y = (float*)(base + z + 2 * h);
   }
-  return z + 2 * h;
+  return z + 2 * h + (own_y ? aligned256((size_t)mp * k.out_dim * sizeof(float)) : 0);
 }
 
-// The networks the allocation-free pass takes: those whose 64 rows of inputs, features, activations,
-// FP32 pre-activations and outputs fit the scratch array.
+// The networks the allocation-free pass takes, wherever y lies: those of which 64 rows of inputs,
+// features, activations, FP32 pre-activations and outputs fit the scratch array. More than a pass keeps
+// there: the limit is the entry point's, the same for every y.
 bool scratch_takes(const Net& n) {
   const dgs_config& k = n.cfg;
   const size_t f = sizeof(float);
-  return aligned256(64 * (size_t)k.in_dim * f) + scratch_layout(n, 64, nullptr, nullptr) +
-             aligned256(64 * (size_t)k.width * f) + aligned256(64 * (size_t)k.out_dim * f) <=
+  return aligned256(64 * (size_t)k.in_dim * f) + scratch_layout(n, 64, true, nullptr, nullptr) +
+             aligned256(64 * (size_t)k.width * f) <=
          kScratchBytes;
+}
+
+// Whether kernels on device dev write p as their own memory: not host memory, which they may have no
+// mapping of, nor another GPU's, which they may have no access to.
+bool own_memory(const void* p, int dev) {
+  hipPointerAttribute_t at;
+  if (hipPointerGetAttributes(&at, p) != hipSuccess) {
+    (void)hipGetLastError();  // memory that the runtime does not know
+    return false;
+  }
+  return at.type == hipMemoryTypeDevice && at.device == dev;
 }
 
 void check_batch(const Net& n, int rows) {
@@ -844,17 +858,20 @@ dgs_status dgs_forward_noalloc(dgs_net* n, int rows, const float* x, float* y) {
     dgs::Pass b{};
     if (!dgs::scratch_takes(*n))
       throw dgs::Error(DGS_ERR_INVALID, "network too wide for the 16 MiB forward scratch (64 rows do not fit)");
+    const bool own_y = rows > 0 && !dgs::own_memory(y, n->device);
     // rows per pass: the largest multiple of 64 whose buffers fit the scratch array
-    int mb = 64 * (int)(dgs::kScratchBytes / dgs::scratch_layout(*n, 64, nullptr, nullptr));
+    const int mb = 64 * (int)(dgs::kScratchBytes / dgs::scratch_layout(*n, 64, own_y, nullptr, nullptr));
     unsigned char* base = dgs::scratch_base(n->device);
     for (int r0 = 0; r0 < rows; r0 += mb) {
       const int m = std::min(mb, rows - r0);
       const int mp = (m + 63) / 64 * 64;  // whole 64-row tiles, padded with copies of the last row
-      dgs::scratch_layout(*n, mp, base, &b);
       b.x = x + (size_t)r0 * in;
       b.m = m;
       b.y = y + (size_t)r0 * No;
+      dgs::scratch_layout(*n, mp, own_y, base, &b);
       dgs::forward(*n, mp, b);
+      if (own_y)
+        DGS_HIP(hipMemcpyAsync(y + (size_t)r0 * No, b.y, (size_t)m * No * sizeof(float), hipMemcpyDefault, n->s));
     }
     DGS_HIP(hipStreamSynchronize(n->s));
   });

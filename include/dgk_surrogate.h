@@ -44,12 +44,13 @@ dgs_status dgs_set_params(dgs_net* net, const float* params, const float* fourie
 /* y[rows][out_dim] = net(x[rows][in_dim]) (host buffers, any row count) */
 dgs_status dgs_forward(dgs_net* net, int rows, const float* x, float* y);
 /* y[rows][out_dim] = net(x[rows][in_dim]) with x and y in device memory of the network's GPU.
- * No counterpart in the reference. For callers that cannot allocate device memory (code under
- * HIP graph capture, tight serving loops): it calls no allocating routine; its activations live
- * in a fixed 16 MiB device array per GPU (rows are processed in passes of the largest multiple
- * of 64 whose activations fit; a network of which 64 rows of inputs, activations and outputs do not
- * fit is rejected with DGS_ERR_INVALID). Ordered on the network's stream and synchronous like dgs_forward. Calls
- * that overlap on one GPU share that array and race. */
+ * No counterpart in the reference. For callers that cannot allocate device memory (tight serving
+ * loops): it calls no allocating routine; its activations live in a fixed 16 MiB device array per GPU
+ * (rows are processed in passes of the largest multiple of 64 that fits). A network of which 64 rows of
+ * inputs, features, activations, pre-activations and outputs do not fit the array is rejected with
+ * DGS_ERR_INVALID. A y elsewhere (host memory, another GPU) is written by copies from the array. Ordered on
+ * the network's stream and synchronous like dgs_forward. Calls that overlap on one GPU share the array and
+ * race. */
 dgs_status dgs_forward_noalloc(dgs_net* net, int rows, const float* x, float* y);
 /* average device time of `reps` forward passes over `rows` rows already on the device: those of the last
  * pass of dgs_forward, dgs_gradients or dgs_train (zero where there was none) */
