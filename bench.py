@@ -59,7 +59,8 @@ def element_sizes(dim, p):
 
 
 def algorithmic_bytes(dim, p, K, F, Fb, word, compensated):
-    """Algorithmic HBM bytes of one stage launch over K elements of one (dim, order).
+    """HBM bytes of one stage launch over K elements of one (dim, order) in the accumulator form, which
+    the stage kernel runs with the compensated solution (stage_bytes has the other forms).
 
     Per counted DOF ((dim+1) fields per node): the stage state traffic averaged over the four
     RK4 stages -- stage 1 reads u and writes the accumulator and the next stage input (3 words),
@@ -77,6 +78,18 @@ def algorithmic_bytes(dim, p, K, F, Fb, word, compensated):
     traces = 2 * (F - Fb) * Nfp * nf * word
     geo = K * (dim * dim * word + Nf * ((dim + 1) * word + 8))
     return dof * state + traces + geo
+
+
+def stage_bytes(dim, p, K, F, Fb, word, compensated):
+    """HBM bytes that one launch of k_stage_mfma moves by its own algorithm, averaged over the four stages.
+
+    With the compensated solution: algorithmic_bytes. Without it no accumulator is kept, and an RK4 step
+    moves 12 state words per DOF instead of 16: stage 1 reads u and writes the next stage input (2), stage
+    2 reads its input and u and writes the next input and the combination that stage 4 needs (4), stage 3
+    reads its input and u and writes the next input (3), stage 4 reads its input and the combination and
+    writes u (3)."""
+    full = algorithmic_bytes(dim, p, K, F, Fb, word, compensated)
+    return full if compensated else full - (dim + 1) * K * element_sizes(dim, p)[0] * word
 
 
 def algorithmic_flops(dim, p, K):
@@ -172,7 +185,7 @@ def single_leg(m, ph, dt, u0, precision, steps, warmup):
     s.close()
     dof = (m.dim + 1) * m.K * m.Np
     word = 8 if precision == dgk.FP64 else 4
-    b = algorithmic_bytes(m.dim, m.order, m.K, info.num_faces, info.num_boundary_faces, word, precision == dgk.FP32)
+    b = stage_bytes(m.dim, m.order, m.K, info.num_faces, info.num_boundary_faces, word, precision == dgk.FP32)
     stage_s = stage_ms * 1e-3 / (4 * nk)
     return dict(rate=dof * 4 * steps / wall, wall=wall, state=state, total_steps=warmup + steps + nk,
                 roofline=roofline(b, algorithmic_flops(m.dim, m.order, m.K), word, stage_s,
@@ -218,7 +231,7 @@ def batch_leg(steps, warmup, members_checked=8, n=256):
     gtab = []
     for g, ms, c in zip(groups, gms, tuned):
         Np = element_sizes(g["dim"], g["order"])[0]
-        bl = algorithmic_bytes(g["dim"], g["order"], g["elements"], g["faces"], g["boundary_faces"], 4, True)
+        bl = stage_bytes(g["dim"], g["order"], g["elements"], g["faces"], g["boundary_faces"], 4, True)
         st = ms * 1e-3 / (4 * nk)
         gtab.append(dict(dim=g["dim"], order=g["order"], sims=g["sims"], elements=g["elements"],
                          tile_shape=c[0], grid_pct=c[1], tile_order=c[2],
