@@ -755,8 +755,10 @@ double* staging(Ctx& c) {
 namespace {
 
 // A state of at most this many bytes goes through a slab that the kernels read and write themselves:
-// no copy commands, whose fixed cost is most of a small hand-over (2D order 2, 2146 elements, 412 KB:
-// dgk_rhs 125 -> 57 us). Half a slab in, half out.
+// no copy commands, whose fixed cost is most of a small hand-over. Half a slab in, half out. us of
+// dgk_set_state / dgk_get_state / dgk_rhs with copies -> without (2D order 3): 0.16 MB 89 / 60 / 146 -> 20 /
+// 20 / 34, 0.84 MB 80 / 77 / 148 -> 51 / 46 / 92, 1.65 MB 106 / 96 / 193 -> 97 / 88 / 169, 2.5 MB 133 / 114 /
+// 239 -> 136 / 124 / 261: the line lies in the safe part of what a slab holds.
 constexpr size_t kDirectBytes = (size_t)1 << 20;
 static_assert(kDirectBytes <= Slabs::kSlabBytes / 2, "a state in and a state out of one slab");
 double* slab_in(Slab& s) { return (double*)s.data(); }

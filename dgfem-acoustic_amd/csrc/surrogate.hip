@@ -491,10 +491,14 @@ void check_gemm(const GemmArgs& g) {
     throw Error(DGS_ERR_INVALID, "GEMM shape must be multiples of 64");
 }
 
-// C = A B with both operands k-contiguous (the forward pass): the largest tile of which there are
-// enough for two or more workgroups per CU, since one alone waits for memory at every K step
-// (6528 x 512 x 512: 204 tiles of 128 take 25.9 us, 816 of 64 14.0 us; 6528 x 2048 x 512: 816 of 128
-// 34 us).
+// C = A B with both operands k-contiguous (the forward pass): the 128-wide tile where there are two
+// workgroups of it per CU (256 of them), the 64-wide one from one and a half per CU on, else the 32-wide.
+// With fewer, a larger tile's workgroups stand alone on their CUs and wait for memory at every K step. us
+// per layer with the 32 / 64 / 128 tile: 2560 x 512 x 512 (320 tiles of 64) 8.5 / 9.4 / 17.6, 3072 (384)
+// 9.5 / 9.6 / 17.7, 4096 (512) 11.3 / 10.0 / 18.0; 12288 x 512 x 512 (384 tiles of 128) 28 / 23.1 / 23.8,
+// 16384 (512) 37 / 28.5 / 25.4, 20480 (640, a last round a quarter full) 45 / 34.9 / 38.7, 8192 x 1024 x
+// 1024 (512) 60 / 40.9 / 33.3.
+constexpr int kTiles128 = 512, kTiles64 = 384;
 template <int EPI>
 void gemm(Net& n, GemmArgs g) {
   check_gemm(g);
@@ -502,8 +506,8 @@ void gemm(Net& n, GemmArgs g) {
   auto cols = [&](int t) { return (g.N + t - 1) / t; };
   auto tiles = [&](int t) { return (int64_t)rows(t) * cols(t); };
   auto grid = [&](int t) { return dim3((rows(t) + 7) / 8 * 8 * cols(t)); };  // row panels in eights, one per XCD
-  if (tiles(128) >= 512) hipLaunchKernelGGL((k_gemm_large<128, EPI>), grid(128), dim3(256), 0, n.s, g);
-  else if (tiles(64) >= 384) hipLaunchKernelGGL((k_gemm_large<64, EPI>), grid(64), dim3(256), 0, n.s, g);
+  if (tiles(128) >= kTiles128) hipLaunchKernelGGL((k_gemm_large<128, EPI>), grid(128), dim3(256), 0, n.s, g);
+  else if (tiles(64) >= kTiles64) hipLaunchKernelGGL((k_gemm_large<64, EPI>), grid(64), dim3(256), 0, n.s, g);
   else
     hipLaunchKernelGGL((k_gemm_small<false, false, EPI>), dim3(cols(kSmall), rows(kSmall)), dim3(256), 0, n.s, g);
   DGS_HIP(hipGetLastError());
@@ -814,8 +818,9 @@ dgs_status dgs_forward(dgs_net* n, int rows, const float* x, float* y) {
   return dgs::guarded(n, [&] {
     const int mb = n->cfg.max_batch, in = n->cfg.in_dim, No = n->cfg.out_dim;
     // few rows: the kernels read the inputs and write the outputs in a page-locked slab themselves (half
-    // of it each), without copy commands (100 rows, 2048 outputs: 124 -> 78 us); otherwise the slab only
-    // carries the inputs
+    // of it each), without copy commands. us with copies / without, 2048 outputs: 16 rows 139 / 47, 64 rows
+    // 105 / 64, 128 rows 138 / 96, 192 rows (1.5 MB) 127 / 124, 256 (2 MB) 149 / 150, 384 187 / 210. More
+    // outputs are downloaded, through the whole slab when its inputs have been read.
     constexpr size_t half = dgk::Slabs::kSlabBytes / 2, most = (size_t)2 << 20;
     static_assert(most <= half, "inputs and outputs of a pass in one slab");
     dgk::Slab slab(n->s);
