@@ -348,12 +348,14 @@ __device__ __forceinline__ uint32_t f32_to_bf16_bits(float f) {
 // Built-in: 8-wave workgroups for 3D order 5 and FP64 3D order 4 (two waves per SIMD share one LDS
 // copy of the operator); for FP64 3D order 5 the 8-wave row split (shape 5: its operator, 110 KB
 // with the compact last row block, fits LDS only beside a small tile); shape 6 for FP32 3D order 4
-// (three 52 KB workgroups per CU); 4-wave workgroups elsewhere.
+// (three 52 KB workgroups per CU); 4-wave workgroups elsewhere, in 1D FP32 with registers for six waves per
+// SIMD (of their own accord they take 80 and five; not with 64-bit addressing, which spills under that
+// budget: 1.2 to 1.5 times the time).
 template <typename T, int D, int P, int SH = 0>
 struct MfmaLaunch {
   static constexpr bool DEF_ROWSPLIT = sizeof(T) == 8 && D == 3 && P == 5;
   static constexpr int DEF_WAVES = (D == 3 && (P == 5 || (P == 4 && sizeof(T) == 8))) ? 8 : 4;
-  static constexpr int DEF_MINW = (sizeof(T) == 4 && D == 3 && P == 4) ? 3 : 1;
+  static constexpr int DEF_MINW = (sizeof(T) == 4 && D == 3 && P == 4) ? 3 : (sizeof(T) == 4 && D == 1) ? 6 : 1;
   static constexpr bool ROWSPLIT = SH == 3 || SH == 5 || (SH == 0 && DEF_ROWSPLIT);
   static constexpr int WAVES = SH == 0 ? DEF_WAVES : (SH == 2 || SH == 5) ? 8 : 4;
   static constexpr int MINW = SH == 0 ? DEF_MINW : (SH >= 6 && SH <= 8) ? SH - 3 : (SH == 9 || SH == 10) ? SH - 5 : SH == 11 ? 3 : 1;
@@ -362,8 +364,10 @@ struct MfmaLaunch {
   static constexpr int KB = 64 * WAVES;              // threads per workgroup
   static constexpr int TE = ROWSPLIT ? WAVES : 4 * WAVES;  // elements per tile (row split: 4 row groups)
   static constexpr int RG = WAVES / (TE / 4);        // row groups: waves sharing one element group
-  // waves that share their elements' work (k_stage_mfma): the workgroup in 2D FP32, one elsewhere
-  static constexpr int GW = RG == 1 && sizeof(T) == 4 && D == 2 ? WAVES : 1;
+  // waves that share their elements' work (k_stage_mfma): the workgroup's in 1D and in FP32 2D, else one
+  static constexpr int GW = RG == 1 && (D == 1 || (D == 2 && sizeof(T) == 4)) ? WAVES : 1;
+  // waves per SIMD that the registers of the kernel with (BIG) or without 64-bit addressing are sized for
+  static constexpr int minw(bool big) { return big && D == 1 ? 1 : MINW; }
 };
 
 // Pad (in values) of the LDS element stride NP*ES. A wave's 4 elements read and write node rows at
@@ -450,7 +454,7 @@ struct MfmaCfg {
 };
 
 template <typename T, int D, int P, bool LO, bool CS, int ES, bool BIG, int SH>
-__global__ __launch_bounds__((MfmaLaunch<T, D, P, SH>::KB), (MfmaLaunch<T, D, P, SH>::MINW)) void k_stage_mfma(
+__global__ __launch_bounds__((MfmaLaunch<T, D, P, SH>::KB), (MfmaLaunch<T, D, P, SH>::minw(BIG))) void k_stage_mfma(
     StageArgs a) {
   static_assert(!CS || sizeof(T) == 4, "the compensated state is an FP32 form");
   using S = Sz<D, P>;
@@ -475,8 +479,11 @@ __global__ __launch_bounds__((MfmaLaunch<T, D, P, SH>::KB), (MfmaLaunch<T, D, P,
   // and the waves of a CU spread over the phases by themselves instead of computing, then waiting,
   // together (five barriers a tile). us per stage (event-timed), workgroup -> wave: FP32 3D order 5,
   // 82,944 elements, 151.6 -> 138.2; FP64 3D order 4, 48,000, 79.1 -> 72.0; FP64 2D order 2, 500,000,
-  // 87.5 -> 85.3; FP32 3D orders 3 and 4 unchanged. 2D FP32, where a wave's 4 elements leave most
-  // lanes of its loads idle, loses 2-3% and keeps the workgroup.
+  // 87.5 -> 85.3; FP32 3D orders 3 and 4 unchanged. Where a wave's 4 elements leave most lanes of its
+  // loads idle the workgroup keeps its elements together: 2D FP32 loses 2-3% otherwise, and 1D (us per
+  // stage in graph replay, wave -> workgroup, with the 1D choices below): order 1, 1,000,000 elements, FP64
+  // 75.5 -> 69.7, FP32 81.9 -> 65.2; order 4, 400,000, FP64 41.4 -> 39.5, FP32 40.1 -> 31.7, and 40,000,
+  // FP32, 5.69 -> 4.99.
   constexpr int GW = MfmaLaunch<T, D, P, SH>::GW, GT = 64 * RG * GW, GE = 4 * GW;
   constexpr int GV = GE * NP * ES / VW;                     // 16-byte vectors of a group's state
   // The state is node-interleaved, [element][node][field] with the ES live fields (nq), so a group's
@@ -500,7 +507,9 @@ __global__ __launch_bounds__((MfmaLaunch<T, D, P, SH>::KB), (MfmaLaunch<T, D, P,
   // when every face node looked up its own face); us per stage before -> after: 3D order 3, 196,608
   // elements, FP32 85.1 -> 73.2, FP64 146 -> 124; 3D order 4, 115,000 elements, FP32 105 -> 94; 2D
   // order 2 FP64, 179,998 elements, 38.2 -> 34.6 (event-timed launches).
-  constexpr int TPF = GT / (GE * NF);
+  // A 1D face has one node, node j of the element on face j, and one thread: with more the others only
+  // repeat its loads (6,666 elements of order 2, FP32, graph replay, 3.26 -> 3.21).
+  constexpr int TPF = D == 1 ? 1 : GT / (GE * NF);
   constexpr int NI = (NFP + TPF - 1) / TPF;                 // face nodes per thread
   typedef typename Mfma<T>::V V;
   constexpr int LES = C::LES;
@@ -591,7 +600,7 @@ __global__ __launch_bounds__((MfmaLaunch<T, D, P, SH>::KB), (MfmaLaunch<T, D, P,
 #pragma unroll
   for (int t = 0; t < NI; ++t) {
     const int k = kk + t * TPF;
-    fo[t] = (fp / NF) * LES + a.fmask[fj * NFP + (k < NFP ? k : NFP - 1)] * ES;
+    fo[t] = (fp / NF) * LES + (D == 1 ? fj : a.fmask[fj * NFP + (k < NFP ? k : NFP - 1)]) * ES;
   }
   auto has_node = [&](int t) { return fact && ((t + 1) * TPF <= NFP || kk + t * TPF < NFP); };
 
