@@ -18,14 +18,15 @@ namespace dgk {
 // Page-locked slabs of kSlabBytes, shared by all contexts and threads of the process: a call takes one
 // for itself and gives it back. At most kSlabsKept wait for the next call, and kSlabsIdle when the last
 // user has left: a program with one context at a time (a loop that creates, runs and destroys) would
-// page-lock anew for each, and page-locking takes 0.2 ms a MB. The size is the least at which a large
-// download is as fast as through more. get_state, one context a call, ms (first call of the process /
-// later calls): 34.6 MB, two slabs of 16 MB freed with the context 8.7 / 7.3 (2.5 where the runtime had
-// kept the memory), 16 MB 6.1 / 2.4, 8 MB 3.3 / 2.4, 4 MB 2.5 / 2.4; 159.7 MB, 16 MB 11.3 / 10.4, 4 MB
-// 11.5 / 10.8. Copies without slabs: 34.6 MB 3.5, 159.7 MB 15.1.
+// page-lock anew for each, and page-locking takes 0.2 ms a MB. The size: what the first large download of
+// a process pays, against what a smaller slab costs each later one. get_state into fresh memory, one
+// context a call, ms (first call of the process / later ones): 34.6 MB, two slabs of 16 MB freed with the
+// context 8.7 / 2.5 or 7.3 (as the runtime kept the memory or not), one of 16 MB 6.1 / 2.4, 8 MB 3.3 / 2.4,
+// 4 MB 2.5 / 2.4; 159.7 MB, 16 MB 11.3 / 10.4, 8 MB 11.2 / 10.5, 4 MB 11.5 / 10.8. Plain copies: 34.6 MB
+// 3.5, 159.7 MB 15.3.
 class Slabs {
  public:
-  static constexpr size_t kSlabBytes = (size_t)4 << 20;
+  static constexpr size_t kSlabBytes = (size_t)8 << 20;
   static constexpr size_t kSlabsKept = 4, kSlabsIdle = 1;
   static Slabs& get() {
     static Slabs* s = new Slabs();  // never destroyed: contexts may outlive static destruction
@@ -116,14 +117,15 @@ struct Piece {
   size_t bytes;
 };
 
-// Copies device pieces to host memory through the call's slab in slots of 1 MB: while slots are in transfer,
-// this thread copies out the one that has landed. Blocks until everything is in place. What the slab held
-// is overwritten, in the order of stream s. The thread polls: one that sleeps gets its core back only at the
+// Copies device pieces to host memory through the call's slab in slots of 2 MB: while slots are in transfer,
+// this thread copies out the one that has landed. (Slots of 1 MB: an uneven ensemble's 16 states, 180 MB,
+// take 0.5-1 ms more beside spinning threads.) Blocks until everything is in place. What the slab held is
+// overwritten, in the order of stream s. The thread polls: one that sleeps gets its core back only at the
 // end of a time slice when the caller's other threads (an OpenMP pool after a loop) spin on all of them, 4 ms
 // a call; for the same reason the copying has no helper threads, which took 3 of 126 MB's 9.5 ms off on a
 // quiet machine and cost 3 ms a call beside spinning ones.
 inline hipError_t download(const std::vector<Piece>& pieces, hipStream_t s, Slab& slab) {
-  constexpr size_t kSlot = (size_t)1 << 20, kSlots = Slabs::kSlabBytes / kSlot;
+  constexpr size_t kSlot = (size_t)2 << 20, kSlots = Slabs::kSlabBytes / kSlot;
   std::vector<Piece> part;
   for (auto& q : pieces)
     for (size_t o = 0; o < q.bytes; o += kSlot)

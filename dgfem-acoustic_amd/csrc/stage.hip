@@ -359,7 +359,7 @@ struct MfmaLaunch {
   static constexpr bool ROWSPLIT = SH == 3 || SH == 5 || (SH == 0 && DEF_ROWSPLIT);
   static constexpr int WAVES = SH == 0 ? DEF_WAVES : (SH == 2 || SH == 5) ? 8 : 4;
   static constexpr int MINW = SH == 0 ? DEF_MINW : (SH >= 6 && SH <= 8) ? SH - 3 : (SH == 9 || SH == 10) ? SH - 5 : SH == 11 ? 3 : 1;
-  static constexpr bool DEFER = SH == 9 || SH == 10 || SH == 11;  // epilogue operands loaded after the volume k-steps  // waves per SIMD the registers are sized for
+  static constexpr bool DEFER = SH == 9 || SH == 10 || SH == 11;  // epilogue operands loaded after the volume k-steps
   static constexpr bool OPG = SH == 4;                // operator fragments from global memory
   static constexpr int KB = 64 * WAVES;              // threads per workgroup
   static constexpr int TE = ROWSPLIT ? WAVES : 4 * WAVES;  // elements per tile (row split: 4 row groups)
@@ -430,7 +430,7 @@ struct MfmaCfg {
   // layouts only, whose element boundaries fall on whole 16-byte vectors) chosen so that the four
   // elements of a wave fall in different LDS banks. A volume k-step's lanes read node 4m+g of their
   // element (16 or 32 bytes) and the result write-out puts row 4g+j (FP32) or g+4j (FP64) of 4
-  // elements x 4 fields: FP32 wants the stride in 4-byte words = 4 mod 16 (or 12), FP64 32 mod 64.
+  // elements x 4 fields: FP32 wants the stride in 4-byte words = 4 or 12 mod 16, FP64 16 or 48 mod 64.
   static constexpr int PADV = lds_pad<T, ES>(NP);
   static constexpr int LES = NP * ES + PADV;
   // face fluxes [element][field][RBP], then the results in the state tile's layout

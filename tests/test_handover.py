@@ -118,7 +118,7 @@ def test_download_that_fails_waits_for_what_is_under_way(tmp_path, at, no_memory
 def test_contexts_one_at_a_time_page_lock_once(tmp_path):
     run(tmp_path, """
   for (int i = 0; i < 10; ++i) { SlabUser u; Slab s(nullptr); assert(s.data()); }
-  assert(allocs == 1 && most_locked <= (size_t)4 << 20);
+  assert(allocs == 1 && most_locked == Slabs::kSlabBytes);
 """)
 
 
