@@ -754,12 +754,13 @@ double* staging(Ctx& c) {
 
 namespace {
 
-// A state of at most this many bytes goes through a slab that the kernels read and write themselves:
-// no copy commands, whose fixed cost is most of a small hand-over. Half a slab in, half out. us of
-// dgk_set_state / dgk_get_state / dgk_rhs with copies -> without (2D order 3): 0.16 MB 89 / 60 / 146 -> 20 /
-// 20 / 34, 0.84 MB 80 / 77 / 148 -> 51 / 46 / 92, 1.65 MB 106 / 96 / 193 -> 97 / 88 / 169, 2.5 MB 133 / 114 /
-// 239 -> 136 / 124 / 261: the line lies in the safe part of what a slab holds.
-constexpr size_t kDirectBytes = (size_t)1 << 20;
+// A state of at most this many bytes goes through a slab that the kernels read and write themselves, in
+// every layout: no copy commands, whose fixed cost is most of a small hand-over, nor the pieces of
+// download(), four of them for a state of any size. Half a slab in, half out. us of dgk_set_state /
+// dgk_get_state / dgk_rhs with copies -> without, interleaved fields (2D order 3): 0.16 MB 89 / 60 / 146 ->
+// 20 / 20 / 34, 0.84 MB 80 / 77 / 148 -> 51 / 46 / 92, 1.65 MB 106 / 96 / 193 -> 97 / 88 / 169, 2.5 MB 133 / 114
+// / 239 -> 136 / 124 / 261.
+constexpr size_t kDirectBytes = (size_t)2 << 20;
 static_assert(kDirectBytes <= Slabs::kSlabBytes / 2, "a state in and a state out of one slab");
 double* slab_in(Slab& s) { return (double*)s.data(); }
 double* slab_out(Slab& s) { return (double*)(s.data() + Slabs::kSlabBytes / 2); }
@@ -769,12 +770,12 @@ bool direct(Slab& s, int64_t n) { return 4 * (size_t)n * sizeof(double) <= kDire
 // Asynchronous: u (or the slab) is read until the stream is synchronised.
 void upload_planes(Ctx& c, const double* u, void* dst, int64_t off, int64_t n, Slab& slab) {
   uint16_t* lo = dst == c.U && c.comp ? c.Ulo : nullptr;
-  if (c.precision == DGK_FP64 && c.es == 1) {  // planes in the state's own precision
-    DGK_HIP(hipMemcpy2DAsync((double*)dst + off, c.PS * sizeof(double), u, n * sizeof(double), n * sizeof(double), 4,
-                             hipMemcpyHostToDevice, c.stream));
-  } else if (direct(slab, n)) {
+  if (direct(slab, n)) {
     memcpy(slab_in(slab), u, 4 * n * sizeof(double));
     state_from_f64(c, slab_in(slab), n, dst, lo, off, n);
+  } else if (c.precision == DGK_FP64 && c.es == 1) {  // planes in the state's own precision
+    DGK_HIP(hipMemcpy2DAsync((double*)dst + off, c.PS * sizeof(double), u, n * sizeof(double), n * sizeof(double), 4,
+                             hipMemcpyHostToDevice, c.stream));
   } else {
     double* s = staging(c) + off;
     DGK_HIP(hipMemcpy2DAsync(s, c.PS * sizeof(double), u, n * sizeof(double), n * sizeof(double), 4,
@@ -787,7 +788,7 @@ void upload_planes(Ctx& c, const double* u, void* dst, int64_t off, int64_t n, S
 void download_planes(Ctx& c, const void* src, double* u, int64_t off, int64_t n, Slab& slab) {
   const uint16_t* lo = src == c.U && c.comp ? c.Ulo : nullptr;
   const int live = c.es > 1 ? c.es : 4;
-  if (c.es > 1 && direct(slab, n)) {
+  if (direct(slab, n)) {
     state_to_f64(c, src, lo, slab_out(slab), n, off, n);
     DGK_HIP(hipStreamSynchronize(c.stream));
     memcpy(u, slab_out(slab), live * n * sizeof(double));

@@ -496,7 +496,7 @@ void check_gemm(const GemmArgs& g) {
 // With fewer, a larger tile's workgroups stand alone on their CUs and wait for memory at every K step. us
 // per layer with the 32 / 64 / 128 tile: 2560 x 512 x 512 (320 tiles of 64) 8.5 / 9.4 / 17.6, 3072 (384)
 // 9.5 / 9.6 / 17.7, 4096 (512) 11.3 / 10.0 / 18.0; 12288 x 512 x 512 (384 tiles of 128) 28 / 23.1 / 23.8,
-// 16384 (512) 37 / 28.5 / 25.4, 20480 (640, a last round a quarter full) 45 / 34.9 / 38.7, 8192 x 1024 x
+// 16384 (512) 37 / 28.5 / 25.4, 20480 (640, the last wave of them a quarter full) 45 / 34.9 / 38.7, 8192 x 1024 x
 // 1024 (512) 60 / 40.9 / 33.3.
 constexpr int kTiles128 = 512, kTiles64 = 384;
 template <int EPI>
